@@ -39,7 +39,9 @@ typedef struct mi_engine mi_engine;
  * SPEC_SLOPE (:1022) -> spec_slope; maxseq = P + n_gen + TMAX (:1023) -> max_ctx. */
 typedef struct mi_opts {
     int32_t max_ctx;       /* KV cache capacity in positions (0: 4096) */
-    int32_t tchunk;        /* prompt tokens per step, 1..8 */
+    int32_t tchunk;        /* prompt tokens per step, 1..8. At 8 (the default) prompts of 17 tokens and more
+                              take panels of up to 512 tokens per pass over the weights instead (same
+                              bits; 512 tokens of the 1.5B shape: 84.1 -> 6.6 ms) */
     int32_t spec;          /* n-gram speculative decoding inside mi_generate: 0 off; 1 the host drafts,
                               launches each verify step and commits its result; 2 the whole loop runs
                               on the device (mega.cu:863-895: each persistent verify launch commits
@@ -92,7 +94,8 @@ int mi_info(const mi_engine* e, mi_model_info* out);
 
 /* Prefill: cuda_infer.cu:1133-1159 / mega.cu:622, 819-820 prompt steps. Runs ids[0..n)
  * at positions 0..n-1 (from an empty cache) in chunks of opts.tchunk tokens (each chunk
- * one multi-token step; results bit-identical to one step per token) and returns the
+ * one multi-token step) or in panels (see tchunk), bit-identical to one step per token
+ * either way, and returns the
  * greedy prediction after the last one (= the first generated token) and its margin. */
 int mi_prefill(mi_engine* e, const int32_t* ids, int32_t n, int32_t* first, float* margin);
 
@@ -130,7 +133,7 @@ int mi_generate(mi_engine* e, int32_t n_gen, int32_t* out, float* margins, int32
 
 /* Teacher forcing: the TEACHER=<k> mode of mega.cu:28-29, 596, 857-862, 1192-1205. Runs
  * ids[0..n) as the context at positions 0..n-1 (from an empty cache) in chunks of
- * opts.tchunk tokens, as mi_prefill does, and returns every position's greedy
+ * opts.tchunk tokens or panels, as mi_prefill does, and returns every position's greedy
  * prediction: pred[i], margin[i] = the argmax (lowest index on ties) and best - second
  * after position i, i.e. the prediction for position i+1. The caller compares
  * pred[i] with ids[i+1] for the positions past its prompt (the reference's "top-1

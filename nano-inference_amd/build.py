@@ -21,7 +21,7 @@ HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contra
              "-Wall", "-Wno-unused-function", "-I", os.path.join(ROOT, "include"), "-I", SRC]
 CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall", "-I", os.path.join(ROOT, "include"), "-I", SRC]
 
-HIP_SOURCES = ["kernels.hip", "engine.hip"]
+HIP_SOURCES = ["kernels.hip", "bulk.hip", "engine.hip"]
 CXX_SOURCES = ["gguf.cpp", "synth.cpp", "spec.cpp", "detok.cpp", "teacher.cpp"]
 
 

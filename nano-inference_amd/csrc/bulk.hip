@@ -1,0 +1,721 @@
+// bulk.hip -- prompt panels (mi_prefill, mi_teacher): up to kBulkM tokens per pass over the
+// weights, one launch per phase (the reference runs its prompt in chunks of up to 8 tokens
+// through forward_batch, cuda_infer.cu:990-1026, 1133-1144; mega.cu:622, 819-820).
+//
+// A prompt in 8-token steps reads the weights once per 8 tokens and pays ~291 grid barriers
+// per step: 1.4 ms a step on the 1.5B shape, 84.1 ms for 512 tokens, 530 ms for 3001. Panels
+// read them once per 512: 6.6 and 53.5 ms.
+//
+// Every value equals the single-token step's bit for bit (the reduction plan at the top of
+// kernels.hip):
+//   q4_0 x int8   the integer block dots on int8 MFMA (exact); dw*dx of a block is an outer
+//                 product, taken by an f32 MFMA of depth 1 (exact: 11 x 11 bits); the fp32
+//                 chain acc = fma(dw*dx, float(dot), acc) stays on the VALU. Chunk sums and
+//                 segments are added left to right as everywhere.
+//   attention     an f32 MFMA is a chain of fused multiply-adds in k order (one rounding per
+//                 term), which is what the canonical q.k and p.v chains are.
+#include "bulk.hpp"
+#include "device.hpp"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace mi {
+
+#define LAUNCH(kern, grid, block, stream, ...) hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, stream, __VA_ARGS__)
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x32 __attribute__((ext_vector_type(32)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int kBMaxE = kMaxE;
+constexpr int kBThreads = 256;
+
+// element offset of (token t, block b, element e of the block) in an operand buffer
+__host__ __device__ __forceinline__ size_t bx_at(int nb, int t, int b, int e) {
+    return ((((size_t)(t >> 5) * nb + b) * 64 + (e >> 4) * 32 + (t & 31)) << 4) + (e & 15);
+}
+__host__ __device__ __forceinline__ size_t bd_at(int nb, int t, int b) { return ((size_t)(t >> 5) * nb + b) * 32 + (t & 31); }
+
+BulkSizes bulk_sizes(int E, int FF, int NH, int HD, int QKV, int V, int maxseq, int ks_d) {
+    const size_t M = kBulkM, nsp = (maxseq + kAttnChunk * kAttnSplit - 1) / (kAttnChunk * kAttnSplit);
+    BulkSizes s;
+    s.h = M * E;
+    s.xq = M * E;
+    s.xd = M * (E / 32);
+    s.qkv = M * QKV;
+    s.aq = M * FF;
+    s.ad = M * (FF / 32);
+    s.dpart = (size_t)ks_d * kBulkSplitM * E;
+    s.rec = M * NH * nsp * (HD + 2);
+    s.cand = M * (V / 64);
+    return s;
+}
+
+// ------------------------------------------------------------------ GEMM
+// D layout of a 32x32 MFMA tile: lane l holds column l % 32, rows 8(j/4) + 4(l/32) + j%4.
+__device__ __forceinline__ int drow(int j, int half) { return 8 * (j >> 2) + 4 * half + (j & 3); }
+
+// 16 nibbles of one half block as int8 16*(n - 8): the low nibbles (elements 0..15) on
+// lanes 0..31, the high ones (16..31) on lanes 32..63. In the byte's upper half and with
+// its top bit flipped a nibble is the signed byte 16(n - 8); the factor 16 comes off with
+// the scale (a power of two, so exactly).
+__device__ __forceinline__ i32x4 unpack16(uint4 w, int sh) {
+    const uint32_t m = 0xF0F0F0F0u, x = 0x80808080u;
+    return i32x4{(int)(((w.x << sh) & m) ^ x), (int)(((w.y << sh) & m) ^ x), (int)(((w.z << sh) & m) ^ x),
+                 (int)(((w.w << sh) & m) ^ x)};
+}
+
+enum BEpi { BE_PART, BE_RES, BE_GU, BE_LM };
+
+struct BStage {                    // one pair of blocks: 64 weight rows, 64 tokens
+    uint4 a[2][2];                 // [32-row tile][block]
+    uint4 b[2][2];                 // [32-token tile][block]
+    float dx[2];                   // token scales: block 2p on lanes 0..31, 2p + 1 on 32..63
+    uint32_t sw[2];                // row scales of both blocks (fp16 x 2), [32-row tile]
+};
+
+// One workgroup: 64 rows x 64 tokens. Wave w takes chunks w, w + 4, ... of the K range: per
+// chunk the 2 x 2 tiles of 32 x 32 outputs run their block chains; then the four waves' chunk
+// sums meet in LDS and wave w adds tile w's in chunk order. Weights and activations go
+// straight to registers (each wave reads its own K range, so there is nothing to share
+// inside the workgroup), one block pair ahead.
+// W: rows of the GEMM; xq/xd: the first token tile; out[..]: token 0 of the first tile.
+// Grid (1-D): XCD x = id % 8 holds row groups g % 8 == x and walks their token tiles next
+// to each other, so a group's weights come from HBM once and are then in that XCD's L2.
+template <int CB, int EPI>
+__global__ __launch_bounds__(kBThreads, 2) void k_bgemm(PMat W, const int8_t* xq, const float* xd, int ntt, int nseg,
+                                                        float* out, int8_t* oq, float4* cand, int ostride) {
+    __shared__ float4 red[4][4][4][64], totl[4][4][64];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, half = lane >> 5, col = lane & 31;
+    const int ng = W.rows >> 6, per = ntt * nseg, id = blockIdx.x;
+    const int k0 = id >> 3, gi = k0 / per, rest = k0 - gi * per, g = gi * 8 + (id & 7);
+    if (g >= ng) return;
+    const int sidx = rest / ntt, tt = rest - sidx * ntt;
+    // K segments [s0, s1) of the plan: all of them, or one per workgroup
+    const int s0 = nseg > 1 ? sidx : 0, s1 = nseg > 1 ? sidx + 1 : W.ks;
+    const int cbeg = s0 * W.nc / W.ks, cend = s1 * W.nc / W.ks;
+    const uint8_t* wbase = W.base + (size_t)g * W.nc * (CB * 1152);
+    const int8_t* xt = xq + (size_t)(2 * tt) * W.nb * 1024 + lane * 16;
+    const float* dt = xd + (size_t)(2 * tt) * W.nb * 32 + lane;
+    const size_t xstep = (size_t)W.nb * 1024, dstep = (size_t)W.nb * 32;
+    const int sh = half ? 0 : 4;
+
+    i32x16 magic;                  // float(1.5 * 2^23 + i) has the bits of 0x4B400000 + i, |i| < 2^22
+#pragma unroll
+    for (int j = 0; j < 16; j++) magic[j] = 0x4B400000;
+    asm volatile("" : "+v"(magic));
+
+    auto load_pair = [&](BStage& s, int c, int p) {
+        const uint8_t* t = wbase + (size_t)c * (CB * 1152) + (2 * p) * 1024 + col * 16;
+        const int b = c * CB + 2 * p;
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            s.a[0][k] = *reinterpret_cast<const uint4*>(t + k * 1024);
+            s.a[1][k] = *reinterpret_cast<const uint4*>(t + k * 1024 + 512);
+            s.b[0][k] = *reinterpret_cast<const uint4*>(xt + (size_t)(b + k) * 1024);
+            s.b[1][k] = *reinterpret_cast<const uint4*>(xt + xstep + (size_t)(b + k) * 1024);
+        }
+        s.dx[0] = dt[(size_t)b * 32];
+        s.dx[1] = dt[dstep + (size_t)b * 32];
+        const uint8_t* ts = wbase + (size_t)c * (CB * 1152) + CB * 1024 + col * (CB * 2) + 4 * p;
+        s.sw[0] = *reinterpret_cast<const uint32_t*>(ts);
+        s.sw[1] = *reinterpret_cast<const uint32_t*>(ts + 32 * CB * 2);
+    };
+    f32x16 acc[2][2];
+    auto pair = [&](const BStage& s) {
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const i32x4 a0 = unpack16(s.a[r][0], sh), a1 = unpack16(s.a[r][1], sh);
+            const uint32_t sw = s.sw[r];
+            const float dw = __fmul_rn(half ? h2f_hi(sw) : h2f_lo(sw), 0.0625f);
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                float dt_ = s.dx[t];
+                asm volatile("" : "+v"(dt_));
+                f32x32 pr = {};
+                pr = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, dt_, pr, 0, 0, 0);
+                uint4 b0 = s.b[t][0], b1 = s.b[t][1];
+                asm volatile("" : "+v"(b0.x), "+v"(b1.x));
+                const i32x16 d0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+                    a0, i32x4{(int)b0.x, (int)b0.y, (int)b0.z, (int)b0.w}, magic, 0, 0, 0);
+                const i32x16 d1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+                    a1, i32x4{(int)b1.x, (int)b1.y, (int)b1.z, (int)b1.w}, magic, 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 16; j++)
+                    acc[r][t][j] = __fmaf_rn(pr[j], __fsub_rn(__int_as_float(d0[j]), 12582912.f), acc[r][t][j]);
+#pragma unroll
+                for (int j = 0; j < 16; j++)
+                    acc[r][t][j] = __fmaf_rn(pr[16 + j], __fsub_rn(__int_as_float(d1[j]), 12582912.f), acc[r][t][j]);
+                asm volatile("" : "+v"(acc[r][t]));          // one tile's products at a time in registers
+            }
+        }
+    };
+
+    BStage st[2];
+    float sg[16];
+#pragma unroll
+    for (int j = 0; j < 16; j++) sg[j] = 0.f;
+    int s = s0, sb = cbeg, se = (s0 + 1) * W.nc / W.ks;      // the segment the sums are in
+    if (cbeg + wave < cend) load_pair(st[0], cbeg + wave, 0);
+    for (int c0 = cbeg; c0 < cend; c0 += 4) {
+        const int c = c0 + wave;
+        if (c < cend) {
+#pragma unroll
+            for (int r = 0; r < 2; r++)
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+#pragma unroll
+                    for (int j = 0; j < 16; j++) acc[r][t][j] = 0.f;
+#pragma unroll
+            for (int p = 0; p < CB / 2; p++) {
+                if (p + 1 < CB / 2) {
+                    load_pair(st[(p + 1) & 1], c, p + 1);
+                } else if (c + 4 < cend) {
+                    load_pair(st[(p + 1) & 1], c + 4, 0);
+                }
+                pair(st[p & 1]);
+            }
+#pragma unroll
+            for (int r = 0; r < 2; r++)
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        red[wave][2 * r + t][j][lane] =
+                            make_float4(acc[r][t][4 * j], acc[r][t][4 * j + 1], acc[r][t][4 * j + 2], acc[r][t][4 * j + 3]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int ci = c0 + i;
+            if (ci < cend) {
+                const bool first = ci == sb;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float4 v = red[i][wave][j][lane];
+                    sg[4 * j] = first ? v.x : __fadd_rn(sg[4 * j], v.x);
+                    sg[4 * j + 1] = first ? v.y : __fadd_rn(sg[4 * j + 1], v.y);
+                    sg[4 * j + 2] = first ? v.z : __fadd_rn(sg[4 * j + 2], v.z);
+                    sg[4 * j + 3] = first ? v.w : __fadd_rn(sg[4 * j + 3], v.w);
+                }
+                if (ci + 1 == se) {                          // segment done: segments left to right
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {            // the lane's own slot, in LDS to spare registers
+                        float4 v = make_float4(sg[4 * j], sg[4 * j + 1], sg[4 * j + 2], sg[4 * j + 3]);
+                        if (s > s0) {
+                            const float4 o = totl[wave][j][lane];
+                            v = make_float4(__fadd_rn(o.x, v.x), __fadd_rn(o.y, v.y), __fadd_rn(o.z, v.z), __fadd_rn(o.w, v.w));
+                        }
+                        totl[wave][j][lane] = v;
+                    }
+                    s++;
+                    sb = se;
+                    se = (s + 1) * W.nc / W.ks;
+                }
+            }
+        }
+        __syncthreads();
+    }
+
+    float tot[16];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const float4 v = totl[wave][j][lane];
+        tot[4 * j] = v.x; tot[4 * j + 1] = v.y; tot[4 * j + 2] = v.z; tot[4 * j + 3] = v.w;
+    }
+    // wave w holds rows 32(w/2).. of the group, tokens 32(w%2).. of the tile
+    const int rt = wave >> 1, tok = (2 * tt + (wave & 1)) * 32 + col;
+    if constexpr (EPI == BE_PART || EPI == BE_RES) {
+        float* o = out + (size_t)sidx * ostride + (size_t)tok * W.rows + g * 64 + rt * 32 + 4 * half;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            float4 v = make_float4(tot[4 * j], tot[4 * j + 1], tot[4 * j + 2], tot[4 * j + 3]);
+            float4* q = reinterpret_cast<float4*>(o + 8 * j);
+            if constexpr (EPI == BE_RES) {
+                const float4 h = *q;
+                v = make_float4(__fadd_rn(h.x, v.x), __fadd_rn(h.y, v.y), __fadd_rn(h.z, v.z), __fadd_rn(h.w, v.w));
+            }
+            *q = v;
+        }
+    } else if constexpr (EPI == BE_GU) {
+        // rows 0..31 of a group are gate rows, 32..63 their up rows: silu(g)*u, then one
+        // int8 block per token
+        if (rt == 1)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                red[0][wave & 1][j][lane] = make_float4(tot[4 * j], tot[4 * j + 1], tot[4 * j + 2], tot[4 * j + 3]);
+        __syncthreads();
+        if (rt == 0) {
+            float a[16], mx = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float4 u = red[0][wave][j][lane];
+                const float uu[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float v = tot[4 * j + i], e = mi_expf(-v);
+                    a[4 * j + i] = __fmul_rn(__fdiv_rn(v, __fadd_rn(1.0f, e)), uu[i]);
+                    mx = fmaxf(mx, fabsf(a[4 * j + i]));
+                }
+            }
+            float x, y;
+            pair32(mx, x, y);
+            mx = fmaxf(x, y);
+            const float inv = mx > 0.f ? __fdiv_rn(127.f, mx) : 0.f;
+            const int nbo = ng;                              // one block per row group
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                uint32_t w = 0;
+#pragma unroll
+                for (int i = 0; i < 4; i++) w |= (uint32_t)(__float2int_rn(__fmul_rn(a[4 * j + i], inv)) & 0xFF) << (8 * i);
+                *reinterpret_cast<uint32_t*>(oq + bx_at(nbo, tok, g, 8 * j + 4 * half)) = w;
+            }
+            if (half == 0) out[bd_at(nbo, tok, g)] = fp16_round(__fdiv_rn(mx, 127.f));
+        }
+    } else {
+        Top2 t{-__builtin_inff(), INT_MAX, -__builtin_inff()};
+#pragma unroll
+        for (int j = 0; j < 16; j++) top2_push(t, tot[j], g * 64 + rt * 32 + drow(j, half));
+        const auto rb = __builtin_amdgcn_permlane32_swap(__float_as_uint(t.best), __float_as_uint(t.best), false, false);
+        const auto ri = __builtin_amdgcn_permlane32_swap((unsigned)t.idx, (unsigned)t.idx, false, false);
+        const auto rs = __builtin_amdgcn_permlane32_swap(__float_as_uint(t.second), __float_as_uint(t.second), false, false);
+        Top2 x{__uint_as_float(rb[0]), (int)ri[0], __uint_as_float(rs[0])};
+        top2_merge(x, __uint_as_float(rb[1]), (int)ri[1], __uint_as_float(rs[1]));
+        if (rt == 1) red[0][wave & 1][0][lane] = make_float4(x.best, __int_as_float(x.idx), x.second, 0.f);
+        __syncthreads();
+        if (rt == 0 && half == 0) {
+            const float4 o = red[0][wave][0][lane];
+            top2_merge(x, o.x, __float_as_int(o.y), o.z);
+            cand[(size_t)tok * ng + g] = make_float4(x.best, __int_as_float(x.idx), x.second, 0.f);
+        }
+    }
+}
+
+// argmax and margin of token t (one wave): the candidates of its V/64 row groups
+__global__ __launch_bounds__(64) void k_bargmax(const float4* cand, int ng, int V, int t0, int p0, int32_t* out_tok,
+                                                float* out_margin) {
+    const int t = t0 + blockIdx.x, lane = threadIdx.x;
+    Top2 a{-__builtin_inff(), INT_MAX, -__builtin_inff()};
+    for (int i = lane; i < ng; i += 64) {
+        const float4 c = cand[(size_t)t * ng + i];
+        top2_merge(a, c.x, __float_as_int(c.y), c.z);
+    }
+    top2_wave(a);
+    if (lane == 0) {
+        out_tok[p0 + t] = top2_token(a, V);
+        out_margin[p0 + t] = __fsub_rn(a.best, a.second);
+    }
+}
+
+// ------------------------------------------------------------------ residual, norm, quant
+// One wave per token: h (layer 0: the embedding row) + the down partials in order, written
+// back; RMSNorm and int8 quantisation into the GEMM operand. Lane l holds elements
+// 256j + 4l .. + 3, the order of the canonical sum of squares (rms_scale).
+__global__ __launch_bounds__(kBThreads) void k_bnorm(int n, float eps, const float* w, float* h, const float* emb,
+                                                     const int32_t* tok, const float* part, int ks, int m, int8_t* xq,
+                                                     float* xd) {
+    constexpr int NJ = kBMaxE / 256;
+    const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (t >= m) return;
+    const float* src = emb ? emb + (size_t)tok[t] * n : h + (size_t)t * n;
+    float4 x[NJ];
+    float a = 0.f;
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        const int e = 256 * j + 4 * lane;
+        x[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (e < n) {
+            x[j] = *reinterpret_cast<const float4*>(src + e);
+            if (ks > 0) {
+                float4 s = *reinterpret_cast<const float4*>(part + (size_t)t * n + e);
+                for (int k = 1; k < ks; k++) {
+                    const float4 p = *reinterpret_cast<const float4*>(part + ((size_t)k * kBulkSplitM + t) * n + e);
+                    s = make_float4(__fadd_rn(s.x, p.x), __fadd_rn(s.y, p.y), __fadd_rn(s.z, p.z), __fadd_rn(s.w, p.w));
+                }
+                x[j] = make_float4(__fadd_rn(x[j].x, s.x), __fadd_rn(x[j].y, s.y), __fadd_rn(x[j].z, s.z),
+                                   __fadd_rn(x[j].w, s.w));
+            }
+            if (emb || ks > 0) *reinterpret_cast<float4*>(h + (size_t)t * n + e) = x[j];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        a = __fmaf_rn(x[j].x, x[j].x, a); a = __fmaf_rn(x[j].y, x[j].y, a);
+        a = __fmaf_rn(x[j].z, x[j].z, a); a = __fmaf_rn(x[j].w, x[j].w, a);
+    }
+    a = bfly_sum64(a);
+    const float sc = __fdiv_rn(1.0f, __builtin_sqrtf(__fadd_rn(__fdiv_rn(a, (float)n), eps)));
+    const int nb = n / 32;
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        if (256 * j >= n) break;
+        const int e = 256 * j + 4 * lane;
+        const bool own = e < n;
+        const float4 wv = own ? *reinterpret_cast<const float4*>(w + e) : make_float4(0.f, 0.f, 0.f, 0.f);
+        float4 y = make_float4(__fmul_rn(__fmul_rn(x[j].x, sc), wv.x), __fmul_rn(__fmul_rn(x[j].y, sc), wv.y),
+                               __fmul_rn(__fmul_rn(x[j].z, sc), wv.z), __fmul_rn(__fmul_rn(x[j].w, sc), wv.w));
+        if (!own) y = make_float4(0.f, 0.f, 0.f, 0.f);
+        const float mx = max8(fmaxf(fmaxf(fabsf(y.x), fabsf(y.y)), fmaxf(fabsf(y.z), fabsf(y.w))));
+        const float inv = mx > 0.f ? __fdiv_rn(127.f, mx) : 0.f;
+        const int q0 = __float2int_rn(__fmul_rn(y.x, inv)), q1 = __float2int_rn(__fmul_rn(y.y, inv));
+        const int q2 = __float2int_rn(__fmul_rn(y.z, inv)), q3 = __float2int_rn(__fmul_rn(y.w, inv));
+        if (own) {
+            *reinterpret_cast<uint32_t*>(xq + bx_at(nb, t, e >> 5, e & 31)) =
+                (uint32_t)(q0 & 0xFF) | ((uint32_t)(q1 & 0xFF) << 8) | ((uint32_t)(q2 & 0xFF) << 16) | ((uint32_t)q3 << 24);
+            if ((lane & 7) == 0) xd[bd_at(nb, t, e >> 5)] = fp16_round(__fdiv_rn(mx, 127.f));
+        }
+    }
+}
+
+// ------------------------------------------------------------------ bias, RoPE, K/V append
+// One thread per (token, head of q|k|v, pair i, i + HD/2): the QKV row + bias, rotated for q
+// (in place) and k; k and v rounded to fp16 into the cache (cpu_infer.cpp:49-61, 114-120).
+template <int HD>
+__global__ __launch_bounds__(kBThreads) void k_brope(float* qkv, const float* bias, const float2* rope, int NH, int NKV,
+                                                     int QKV, int m, int p0, int maxseq, __half* kc, __half* vc) {
+    constexpr int half = HD / 2;
+    const int nh = NH + 2 * NKV;
+    const size_t id = (size_t)blockIdx.x * kBThreads + threadIdx.x;
+    const int i = (int)(id % half), h = (int)((id / half) % nh), t = (int)(id / half / nh);
+    if (t >= m) return;
+    float* r = qkv + (size_t)t * QKV + h * HD;
+    const float x0 = __fadd_rn(r[i], bias[h * HD + i]), x1 = __fadd_rn(r[i + half], bias[h * HD + i + half]);
+    if (h >= NH + NKV) {
+        __half* d = vc + ((size_t)(h - NH - NKV) * maxseq + p0 + t) * HD;
+        d[i] = __float2half(x0);
+        d[i + half] = __float2half(x1);
+        return;
+    }
+    const float2 cz = rope[(size_t)(p0 + t) * half + i];
+    const float y0 = __fsub_rn(__fmul_rn(x0, cz.x), __fmul_rn(x1, cz.y));
+    const float y1 = __fadd_rn(__fmul_rn(x0, cz.y), __fmul_rn(x1, cz.x));
+    if (h < NH) {
+        r[i] = y0;
+        r[i + half] = y1;
+    } else {
+        __half* d = kc + ((size_t)(h - NH) * maxseq + p0 + t) * HD;
+        d[i] = __float2half(y0);
+        d[i + half] = __float2half(y1);
+    }
+}
+
+// ------------------------------------------------------------------ attention
+// One workgroup: 32 tokens of one query head against one split (16 chunks of 64 positions).
+// Wave w takes chunks w, w + 4, ...: scores S[position][token] by 32x32x2 f32 MFMAs, one
+// accumulator per chain d mod 4 (k = 0, 1 of an MFMA are d and d + 4 of a chain), the chunk
+// softmax in registers (lane l: token l % 32, half of the chunk's positions; the other half
+// on lane l ^ 32), and, once every chunk's max is known, o[dim][token] by MFMAs over
+// position pairs. The four waves' chunk outputs meet in LDS per round and are merged in
+// chunk order. Rows of D stand for dims NDT*row + dt, so that one lane's V operands of a
+// position are NDT consecutive halves.
+// Record of (token, head, split): o[HD], M, den.
+template <int HD>
+__global__ __launch_bounds__(kBThreads, 1) void k_battn(const float* qkv, int QKV, const __half* kc, const __half* vc,
+                                                        int NH, int G, int m, int p0, int maxseq, int nsp, float scale,
+                                                        float* rec) {
+    constexpr int NJ = HD / 8, NDT = HD / 32;
+    constexpr int kR = kAttnSplit / 4;                       // rounds of four chunks
+    __shared__ float4 ol[4][NDT][4][64];
+    __shared__ float mt[kAttnSplit][32], lt[kAttnSplit][32];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, half = lane >> 5, col = lane & 31;
+    const int ntile = (m + 31) / 32;
+    // the last (longest) tiles first
+    const int h = blockIdx.x % NH, rest = blockIdx.x / NH, sp = rest % nsp, tile = ntile - 1 - rest / nsp;
+    const int tbase = tile * 32, tlast = min(tbase + 31, m - 1);
+    const int nch = (p0 + tlast) / kAttnChunk + 1 - sp * kAttnSplit;    // chunks of this split, if positive
+    if (nch <= 0) return;
+    const int nc = min(nch, kAttnSplit), nr = (nc + 3) / 4;
+    const int tok = min(tbase + col, tlast), pos = p0 + tok, kvh = h / G, prow = p0 + m - 1;
+    const __half* kb = kc + (size_t)kvh * maxseq * HD;
+    const __half* vb = vc + (size_t)kvh * maxseq * HD;
+
+    float q[NJ][4];                                          // q[token][8j + 4 half + i]
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        const float4 v = *reinterpret_cast<const float4*>(qkv + (size_t)tok * QKV + h * HD + 8 * j + 4 * half);
+        q[j][0] = v.x; q[j][1] = v.y; q[j][2] = v.z; q[j][3] = v.w;
+    }
+    float p[kR][2][16];                                      // scores, then probabilities, of the wave's chunks
+#pragma unroll
+    for (int r = 0; r < kR; r++) {
+        const int ci = 4 * r + wave;
+        if (ci < nc) {
+            const int t0 = (sp * kAttnSplit + ci) * kAttnChunk;
+            f32x16 s[2][4];
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) s[u][i] = f32x16{};
+            const __half* k0 = kb + (size_t)min(t0 + col, prow) * HD + 4 * half;
+            const __half* k1 = kb + (size_t)min(t0 + 32 + col, prow) * HD + 4 * half;
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                const uint2 a = *reinterpret_cast<const uint2*>(k0 + 8 * j);
+                const uint2 b = *reinterpret_cast<const uint2*>(k1 + 8 * j);
+                const float av[4] = {h2f_lo(a.x), h2f_hi(a.x), h2f_lo(a.y), h2f_hi(a.y)};
+                const float bv[4] = {h2f_lo(b.x), h2f_hi(b.x), h2f_lo(b.y), h2f_hi(b.y)};
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    s[0][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], q[j][i], s[0][i], 0, 0, 0);
+                    s[1][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[i], q[j][i], s[1][i], 0, 0, 0);
+                }
+            }
+            float mx = -__builtin_inff();
+            bool any = false;
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int j = 0; j < 16; j++) {
+                    const bool ok = t0 + 32 * u + drow(j, half) <= pos;
+                    const float v = __fmul_rn(__fadd_rn(__fadd_rn(s[u][0][j], s[u][1][j]), __fadd_rn(s[u][2][j], s[u][3][j])), scale);
+                    p[r][u][j] = ok ? v : -__builtin_inff();
+                    mx = any ? fmaxf(mx, p[r][u][j]) : p[r][u][j];
+                    any = true;
+                }
+            float x, y;
+            pair32(mx, x, y);
+            mx = fmaxf(x, y);
+            float e1[2][16];
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int j = 0; j < 16; j++) {
+                    const bool ok = t0 + 32 * u + drow(j, half) <= pos;
+                    p[r][u][j] = ok ? mi_expf(__fsub_rn(p[r][u][j], mx)) : 0.f;
+                    e1[u][j] = p[r][u][j];
+                }
+            // the canonical butterfly over positions: xor 32 (u), 16 and 8 (j / 4), 4 (lane
+            // half), 2 and 1 (j % 4)
+            float b4[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                float z[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) z[j] = __fadd_rn(e1[0][4 * j + i], e1[1][4 * j + i]);
+                const float y0 = __fadd_rn(z[0], z[2]), y1 = __fadd_rn(z[1], z[3]);
+                pair32(__fadd_rn(y0, y1), x, y);
+                b4[i] = __fadd_rn(x, y);
+            }
+            const float ls = __fadd_rn(__fadd_rn(b4[0], b4[2]), __fadd_rn(b4[1], b4[3]));
+            if (half == 0) {
+                mt[ci][col] = mx;
+                lt[ci][col] = ls;
+            }
+        }
+    }
+    __syncthreads();
+    // this token's chunks of the split, their max, and the merge in chunk order
+    const int nct = min(pos / kAttnChunk + 1 - sp * kAttnSplit, kAttnSplit);     // may be <= 0 for the tile's first tokens
+    float Ms = mt[0][col];
+#pragma unroll
+    for (int c = 1; c < kAttnSplit; c++)
+        if (c < nct) Ms = fmaxf(Ms, mt[c][col]);
+    float den = 0.f, as[4 * NDT];
+#pragma unroll
+    for (int j = 0; j < 4 * NDT; j++) as[j] = 0.f;
+#pragma unroll
+    for (int r = 0; r < kR; r++) {
+        if (r < nr) {
+            const int ci = 4 * r + wave;
+            if (ci < nc) {
+                const int t0 = (sp * kAttnSplit + ci) * kAttnChunk;
+                f32x16 o[NDT];
+#pragma unroll
+                for (int d = 0; d < NDT; d++) o[d] = f32x16{};
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        // positions 32u + 8j .. + 7: half 0 holds 0..3, half 1 4..7; the MFMA
+                        // wants pairs (0,1), (2,3), (4,5), (6,7) across the halves
+                        const auto sa = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[r][u][4 * j]), __float_as_uint(p[r][u][4 * j + 1]), false, false);
+                        const auto sb = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[r][u][4 * j + 2]), __float_as_uint(p[r][u][4 * j + 3]), false, false);
+                        const float pb[4] = {__uint_as_float(sa[0]), __uint_as_float(sb[0]), __uint_as_float(sa[1]), __uint_as_float(sb[1])};
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            const int row = min(t0 + 32 * u + 8 * j + 2 * i + half, prow);
+                            const __half* v = vb + (size_t)row * HD + NDT * col;
+                            float vv[NDT];
+                            if constexpr (NDT == 4) {
+                                const uint2 w = *reinterpret_cast<const uint2*>(v);
+                                vv[0] = h2f_lo(w.x); vv[1] = h2f_hi(w.x); vv[2] = h2f_lo(w.y); vv[3] = h2f_hi(w.y);
+                            } else {
+                                const uint32_t w = *reinterpret_cast<const uint32_t*>(v);
+                                vv[0] = h2f_lo(w); vv[1] = h2f_hi(w);
+                            }
+#pragma unroll
+                            for (int d = 0; d < NDT; d++) o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[d], pb[i], o[d], 0, 0, 0);
+                        }
+                    }
+                // A position past a token's own has p = 0, which adds exactly nothing unless its V
+                // holds an infinity or NaN (0 * inf): the canonical chain stops before it. So where
+                // the chunk reaches past the tile's first token and a result is NaN, the chain runs
+                // again one position at a time, each result kept only for the tokens that see it.
+                if (t0 + kAttnChunk - 1 > p0 + tbase) {
+                    bool nan = false;
+#pragma unroll
+                    for (int d = 0; d < NDT; d++)
+#pragma unroll
+                        for (int j = 0; j < 16; j++) nan |= o[d][j] != o[d][j];
+                    if (__builtin_amdgcn_ballot_w64(nan)) {
+                        float* ps = reinterpret_cast<float*>(&ol[wave][0][0][0]);       // [64 positions][32 tokens]
+#pragma unroll
+                        for (int u = 0; u < 2; u++)
+#pragma unroll
+                            for (int j = 0; j < 16; j++) ps[(32 * u + drow(j, half)) * 32 + col] = p[r][u][j];
+                        __builtin_amdgcn_s_waitcnt(0xC07F);
+#pragma unroll
+                        for (int d = 0; d < NDT; d++) o[d] = f32x16{};
+#pragma unroll 1
+                        for (int k = 0; k < kAttnChunk; k++) {
+                            const bool on = (k & 1) == half, sees = t0 + k <= pos;
+                            const float pk = on ? ps[k * 32 + col] : 0.f;
+                            const __half* v = vb + (size_t)min(t0 + k, prow) * HD + NDT * col;
+#pragma unroll
+                            for (int d = 0; d < NDT; d++) {
+                                const f32x16 z = __builtin_amdgcn_mfma_f32_32x32x2f32(on ? __half2float(v[d]) : 0.f, pk, o[d], 0, 0, 0);
+#pragma unroll
+                                for (int j = 0; j < 16; j++) o[d][j] = sees ? z[j] : o[d][j];
+                            }
+                        }
+                        __builtin_amdgcn_s_waitcnt(0xC07F);
+                    }
+                }
+#pragma unroll
+                for (int d = 0; d < NDT; d++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        ol[wave][d][j][lane] = make_float4(o[d][4 * j], o[d][4 * j + 1], o[d][4 * j + 2], o[d][4 * j + 3]);
+            }
+            __syncthreads();
+            // wave w merges quarter w of the 4 NDT float4 a lane holds
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int c = 4 * r + i;
+                if (c < nct) {
+                    const float wc = mi_expf(__fsub_rn(mt[c][col], Ms));
+                    den = __fmaf_rn(lt[c][col], wc, den);
+#pragma unroll
+                    for (int k = 0; k < NDT; k++) {
+                        const int f = wave * NDT + k;
+                        const float4 v = ol[i][f >> 2][f & 3][lane];
+                        as[4 * k] = __fmaf_rn(v.x, wc, as[4 * k]);
+                        as[4 * k + 1] = __fmaf_rn(v.y, wc, as[4 * k + 1]);
+                        as[4 * k + 2] = __fmaf_rn(v.z, wc, as[4 * k + 2]);
+                        as[4 * k + 3] = __fmaf_rn(v.w, wc, as[4 * k + 3]);
+                    }
+                }
+            }
+            __syncthreads();
+        }
+    }
+    if (tbase + col > tlast || nct <= 0) return;
+    float* rp = rec + (((size_t)tok * NH + h) * nsp + sp) * (HD + 2);
+#pragma unroll
+    for (int k = 0; k < NDT; k++) {
+        const int f = wave * NDT + k, d = f >> 2, j = f & 3;
+#pragma unroll
+        for (int i = 0; i < 4; i++) rp[NDT * (8 * j + 4 * half + i) + d] = as[4 * k + i];
+    }
+    if (wave == 0 && half == 0) {
+        rp[HD] = Ms;
+        rp[HD + 1] = den;
+    }
+}
+
+// split merge of (token, head) by one wave (lane = dims 64e + lane), then int8 blocks into
+// the O GEMM's operand
+template <int HD>
+__global__ __launch_bounds__(kBThreads) void k_bcomb(const float* rec, int NH, int m, int p0, int nsp, int nb, int8_t* xq,
+                                                     float* xd) {
+    constexpr int DPL = HD / 64;
+    const int item = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (item >= m * NH) return;
+    const int t = item / NH, h = item - t * NH;
+    const int ns = (p0 + t) / (kAttnChunk * kAttnSplit) + 1;
+    const float* r = rec + (size_t)item * nsp * (HD + 2);
+    float den, o[DPL];
+    if (ns == 1) {
+        den = r[HD + 1];
+#pragma unroll
+        for (int e = 0; e < DPL; e++) o[e] = r[64 * e + lane];
+    } else {
+        float Mx = -__builtin_inff();
+        for (int s = lane; s < ns; s += 64) Mx = fmaxf(Mx, r[(size_t)s * (HD + 2) + HD]);
+        Mx = wave_max(Mx);
+        den = 0.f;
+#pragma unroll
+        for (int e = 0; e < DPL; e++) o[e] = 0.f;
+        for (int s = 0; s < ns; s++) {
+            const float* q = r + (size_t)s * (HD + 2);
+            const float w = mi_expf(__fsub_rn(q[HD], Mx));
+            den = __fmaf_rn(q[HD + 1], w, den);
+#pragma unroll
+            for (int e = 0; e < DPL; e++) o[e] = __fmaf_rn(q[64 * e + lane], w, o[e]);
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < DPL; e++) {
+        int q, s8;
+        float d;
+        quant32_vals(__fdiv_rn(o[e], den), q, d, s8);
+        const int el = h * HD + 64 * e + lane;
+        const uint32_t b = (uint32_t)(q & 0xFF);
+        const uint32_t wd = b | (__shfl_down(b, 1) << 8) | (__shfl_down(b, 2) << 16) | (__shfl_down(b, 3) << 24);
+        if ((lane & 3) == 0) *reinterpret_cast<uint32_t*>(xq + bx_at(nb, t, el >> 5, el & 31)) = wd;
+        if ((lane & 31) == 0) xd[bd_at(nb, t, el >> 5)] = d;
+    }
+}
+
+// ------------------------------------------------------------------ host side
+template <int EPI>
+static void gemm(const PMat& W, const int8_t* xq, const float* xd, int ntt, int nseg, float* out, int8_t* oq, float4* cand,
+                 int ostride, hipStream_t s) {
+    const int grid = 8 * (((W.rows >> 6) + 7) / 8) * ntt * nseg;
+    if (W.cb == 8) LAUNCH((k_bgemm<8, EPI>), grid, kBThreads, s, W, xq, xd, ntt, nseg, out, oq, cand, ostride);
+    else LAUNCH((k_bgemm<4, EPI>), grid, kBThreads, s, W, xq, xd, ntt, nseg, out, oq, cand, ostride);
+}
+
+void launch_bulk(const DModel& M, const DLayer* layers, const BulkBuf& B, int p0, int m, bool all, bool last,
+                 hipStream_t s) {
+    const int E = M.E, ntt = (m + 63) / 64, nbE = E / 32;
+    const int nsp = (p0 + m - 1) / (kAttnChunk * kAttnSplit) + 1;
+    auto norm = [&](const float* w, const float* emb, int ks) {
+        LAUNCH(k_bnorm, (m + 3) / 4, kBThreads, s, E, M.eps, w, B.h, emb, M.tokbuf + p0, B.dpart, ks, m, B.xq, B.xd);
+    };
+    int ks = 0;                                              // down partials the next norm adds
+    for (int l = 0; l < M.NL; l++) {
+        const DLayer& L = layers[l];
+        norm(L.an, l == 0 ? M.emb : nullptr, ks);
+        gemm<BE_PART>(L.qkv, B.xq, B.xd, ntt, 1, B.qkv, nullptr, nullptr, 0, s);
+        const size_t kv = (size_t)l * M.NKV * M.maxseq * M.HD;
+        auto attn = [&](auto hd) {
+            constexpr int HD = decltype(hd)::value;
+            const size_t threads = (size_t)m * (M.NH + 2 * M.NKV) * (HD / 2);
+            LAUNCH((k_brope<HD>), (unsigned)((threads + kBThreads - 1) / kBThreads), kBThreads, s, B.qkv, L.bqkv, M.rope, M.NH,
+                   M.NKV, M.QKV, m, p0, M.maxseq, M.kc + kv, M.vc + kv);
+            LAUNCH((k_battn<HD>), (unsigned)(M.NH * nsp * ((m + 31) / 32)), kBThreads, s, B.qkv, M.QKV, M.kc + kv, M.vc + kv,
+                   M.NH, M.G, m, p0, M.maxseq, nsp, M.scale, B.rec);
+            LAUNCH((k_bcomb<HD>), (m * M.NH + 3) / 4, kBThreads, s, B.rec, M.NH, m, p0, nsp, nbE, B.xq, B.xd);
+        };
+        if (M.HD == 64) attn(std::integral_constant<int, 64>());
+        else attn(std::integral_constant<int, 128>());
+        gemm<BE_RES>(L.o, B.xq, B.xd, ntt, 1, B.h, nullptr, nullptr, 0, s);
+        norm(L.fn, nullptr, 0);
+        gemm<BE_GU>(L.gu, B.xq, B.xd, ntt, 1, B.ad, B.aq, nullptr, 0, s);
+        ks = ntt * 64 <= kBulkSplitM ? L.d.ks : 0;
+        if (ks) gemm<BE_PART>(L.d, B.aq, B.ad, ntt, ks, B.dpart, nullptr, nullptr, kBulkSplitM * E, s);
+        else gemm<BE_RES>(L.d, B.aq, B.ad, ntt, 1, B.h, nullptr, nullptr, 0, s);
+    }
+    if (!all && !last) return;
+    norm(M.out_norm, nullptr, ks);
+    // predictions: every token tile, or only the one that holds the last token
+    const int tt0 = all ? 0 : ntt - 1, t0 = all ? 0 : m - 1;
+    gemm<BE_LM>(M.lm, B.xq + (size_t)(2 * tt0) * nbE * 1024, B.xd + (size_t)(2 * tt0) * nbE * 32, ntt - tt0, 1, nullptr, nullptr,
+                B.cand + (size_t)tt0 * 64 * (M.V / 64), 0, s);
+    LAUNCH(k_bargmax, m - t0, 64, s, B.cand, M.V / 64, M.V, t0, p0, M.out_tok, M.out_margin);
+}
+
+}  // namespace mi

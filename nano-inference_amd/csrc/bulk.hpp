@@ -1,0 +1,39 @@
+// bulk.hpp -- prompt panels: up to kBulkM consecutive tokens through every layer at once
+// (bulk.hip). Used by mi_prefill and mi_teacher; results equal one step per token bit for
+// bit.
+#pragma once
+#include "kernels.hpp"
+
+namespace mi {
+
+constexpr int kBulkM = 512;        // tokens of one panel, a multiple of 64
+// Shorter prompts stay with 8-token steps (1.4 ms each on the 1.5B shape, 0.98 on the 0.5B
+// one): a panel of 17 tokens takes 3.2 / 2.0 ms, three steps 4.2 / 2.9, two steps 2.8 / 2.0.
+constexpr int kBulkMin = 17;
+constexpr int kBulkSplitM = 128;   // up to this many tokens the down GEMM runs one workgroup per K segment
+
+// Work buffers of a panel (device memory, kept by the engine). Int8 activations of an
+// nb-block vector per token are stored as the GEMM's MFMA operand: 32-token tiles, per tile
+// and block 64 lanes x 16 codes (lane l: token l % 32, elements 16 (l / 32) .. + 15), with
+// the block scales [tile][nb][32] beside them.
+struct BulkBuf {
+    float* h;                      // [kBulkM][E] residual
+    int8_t* xq;                    // [kBulkM/32][E/32][64][16]
+    float* xd;                     // [kBulkM/32][E/32][32]
+    float* qkv;                    // [kBulkM][QKV] projections, then q rotated in place
+    int8_t* aq;                    // [kBulkM/32][FF/32][64][16] gate/up output
+    float* ad;                     // [kBulkM/32][FF/32][32]
+    float* dpart;                  // [ks of down][kBulkSplitM][E]
+    float* rec;                    // [kBulkM][NH][max splits][HD + 2] attention split records
+    float4* cand;                  // [kBulkM][V/64] argmax candidates
+};
+struct BulkSizes { size_t h, xq, xd, qkv, aq, ad, dpart, rec, cand; };   // in elements
+BulkSizes bulk_sizes(int E, int FF, int NH, int HD, int QKV, int V, int maxseq, int ks_d);
+
+// tokens tokbuf[p0 .. p0+m-1] (m <= kBulkM) at positions p0..: K/V appended to the cache.
+// all: every position's prediction goes to out_tok / out_margin; otherwise, when last is
+// set, only the last position's. layers: the host copy of M.layers.
+void launch_bulk(const DModel& M, const DLayer* layers, const BulkBuf& B, int p0, int m, bool all, bool last,
+                 hipStream_t s);
+
+}  // namespace mi

@@ -7,6 +7,7 @@
 // allocate the fp16 KV cache and the step's work buffers. Steps then run on one HIP
 // stream without host round trips: the token of each position lives in device
 // memory (tokbuf), and each step's argmax writes the next token there.
+#include "bulk.hpp"
 #include "common.hpp"
 #include "gguf.hpp"
 #include "kernels.hpp"
@@ -46,6 +47,8 @@ struct mi_engine {
     DModel M_logits{};            // same as M with the logits buffer attached
     DModel* dM = nullptr;         // device copies the kernels read: [0] M, [1] M_logits, [2] profiling
     DLayer* d_layers = nullptr;
+    std::vector<DLayer> layers;   // host copy (the panel launches take the matrices as arguments)
+    BulkBuf bulk{};               // work buffers of the prompt panels
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int nwg_persistent = 0;       // workgroups of the persistent step kernel (0: per-phase launches)
@@ -383,7 +386,8 @@ static int load_impl(mi_engine* e, const char* path) {
     if (te->cols() != e->E || te->rows() < e->V || tout->cols() != e->E || tout->rows() != e->V)
         return set_err(e, MI_ERR_FORMAT, "embedding/output shapes do not match the metadata");
 
-    std::vector<DLayer> layers(e->NL);
+    std::vector<DLayer>& layers = e->layers;
+    layers.resize(e->NL);
     std::vector<uint8_t> cat;
     const size_t rbE = (size_t)nbE * 18, rbF = (size_t)nbF * 18;
     for (int l = 0; l < e->NL; l++) {
@@ -514,6 +518,14 @@ static int load_impl(mi_engine* e, const char* path) {
         (rc = alloc_buf(e, &M.actT, lay::actT_size(D))) ||
         (rc = alloc_buf(e, &M.dT, lay::dT_size(D))) ||
         (rc = alloc_buf(e, &M.candT, lay::candT_size(D))) || (rc = alloc_buf(e, &M.spec, 1)))
+        return rc;
+    // prompt panels (mi_prefill, mi_teacher)
+    const BulkSizes bs = bulk_sizes(e->E, e->FF, e->NH, e->HD, e->QKV, e->V, e->maxseq, e->ks[3]);
+    BulkBuf& B = e->bulk;
+    if ((rc = alloc_buf(e, &B.h, bs.h)) || (rc = alloc_buf(e, &B.xq, bs.xq)) || (rc = alloc_buf(e, &B.xd, bs.xd)) ||
+        (rc = alloc_buf(e, &B.qkv, bs.qkv)) || (rc = alloc_buf(e, &B.aq, bs.aq)) || (rc = alloc_buf(e, &B.ad, bs.ad)) ||
+        (rc = alloc_buf(e, &B.dpart, bs.dpart)) || (rc = alloc_buf(e, &B.rec, bs.rec)) ||
+        (rc = alloc_buf(e, &B.cand, bs.cand)))
         return rc;
     M.logits = nullptr;
     M.logitsT = nullptr;
@@ -920,6 +932,20 @@ static int generate_ring(mi_engine* e, int n_gen, int32_t* out, float* margins, 
     return MI_OK;
 }
 
+// Prompts of kBulkMin tokens and more go through the weights in panels of up to kBulkM
+// tokens (bulk.hip; the same bits). tchunk below its maximum asks for smaller steps and
+// keeps them.
+static bool use_bulk(const mi_engine* e, int n) { return n >= kBulkMin && e->opts.tchunk == kMaxT; }
+static int run_bulk(mi_engine* e, int n, bool all) {
+    const int np = (n + kBulkM - 1) / kBulkM, per = ((n + np - 1) / np + 63) / 64 * 64;   // even panels, whole tiles
+    for (int p = 0; p < n; p += per) {
+        const int m = std::min(per, n - p);
+        launch_bulk(e->M, e->layers.data(), e->bulk, p, m, all, p + m == n, e->stream);
+        HIPCHK(e, hipGetLastError());
+    }
+    return MI_OK;
+}
+
 extern "C" {
 
 int mi_step(mi_engine* e, const int32_t* toks, int32_t T, int32_t pos, int32_t* argmax, float* margin, float* logits) {
@@ -967,7 +993,10 @@ int mi_prefill(mi_engine* e, const int32_t* ids, int32_t n, int32_t* first, floa
     HIPCHK(e, hipEventRecord(e->ev0, e->stream));
     // chunks of tchunk tokens through the multi-token step (cuda_infer.cu:1133-1144,
     // mega.cu:622, 819-820); its results equal one step per token bit for bit
-    for (int p = 0; p < n;) {
+    if (use_bulk(e, n)) {
+        if (int rc = run_bulk(e, n, false)) return rc;
+        HIPCHK(e, hipMemcpyAsync(e->M.tokbuf + n, e->M.out_tok + n - 1, 4, hipMemcpyDeviceToDevice, e->stream));
+    } else for (int p = 0; p < n;) {
         const int T = std::min(e->opts.tchunk, n - p);
         if (T == 1) {
             if (int rc = run_step(e, p, p == n - 1, false)) return rc;
@@ -1004,7 +1033,9 @@ int mi_teacher(mi_engine* e, const int32_t* ids, int32_t n, int32_t* pred, float
     for (int i = 0; i < n; i++)
         if (ids[i] < 0 || ids[i] >= e->V) return set_err(e, MI_ERR_ARG, "teacher token %d out of range", ids[i]);
     HIPCHK(e, hipMemcpyAsync(e->M.tokbuf, ids, sizeof(int32_t) * n, hipMemcpyHostToDevice, e->stream));
-    for (int p = 0; p < n;) {
+    if (use_bulk(e, n)) {
+        if (int rc = run_bulk(e, n, true)) return rc;
+    } else for (int p = 0; p < n;) {
         const int T = std::min(e->opts.tchunk, n - p);
         if (T == 1) {
             if (int rc = run_step(e, p, 0, false)) return rc;

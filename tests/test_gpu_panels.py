@@ -1,0 +1,90 @@
+"""GPU parity of the prompt panels (csrc/bulk.hip): mi_prefill and mi_teacher run prompts of
+17 tokens and more in panels of up to 512 tokens. Bar: the same bits as one multi-token step
+per 7 tokens (tchunk=7, itself bit-identical to single steps and the q8act oracle), in the
+predictions, the margins and, through a step's logits, the K/V the panel left.
+
+Lengths sit on the edges of the 32-token tiles, the 64-token GEMM tiles, the panel whose down
+matrix is split over workgroups (128), the panel (512) and the attention split (1024)."""
+import sys
+
+import numpy as np
+import pytest
+
+import minfer
+from conftest import gguf_tensor, synth_cached
+
+pytestmark = pytest.mark.gpu
+# head size 64 with chunks of 8 blocks; head size 128, 7 query heads per kv head, chunks of 4
+TINY = dict(n_layer=2, n_embd=256, n_ff=512, n_head=4, n_head_kv=2, n_vocab=4096)
+ODD = dict(n_layer=2, n_embd=896, n_ff=1152, n_head=7, n_head_kv=1, n_vocab=4160)
+SHAPES = {"hd64": TINY, "hd128-cb4": ODD}
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+
+
+def bits(x):
+    return np.asarray(x, np.float32).view(np.uint32)
+
+
+@pytest.fixture(scope="module", params=list(SHAPES))
+def pair(request):
+    """an engine that runs panels and one that runs 7-token steps, the same model"""
+    shape = SHAPES[request.param]
+    path = synth_cached("panel-" + request.param, shape, 31, qk_bias_std=2.0, norm_offset=1.0)
+    a, b = minfer.Engine(path, max_ctx=1152), minfer.Engine(path, max_ctx=1152, tchunk=7)
+    yield shape, a, b
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("n", [17, 32, 33, 63, 64, 65, 128, 129, 257, 512, 513, 1024, 1025, 1151])
+def test_panel_bit_identical(pair, n):
+    shape, a, b = pair
+    print("[gpu-panel] n", n, flush=True)
+    ids = minfer.prompt_ids(n, n, shape["n_vocab"])
+    pa, ma = a.teacher(ids)
+    pb, mb = b.teacher(ids)
+    assert pa == pb and np.array_equal(bits(ma), bits(mb))
+    fa, fb = a.prefill(ids), b.prefill(ids)
+    assert fa[0] == fb[0] == pb[-1] and bits(fa[1]) == bits(fb[1])
+    _, _, la = a.step(ids[0], n, want_logits=True)
+    _, _, lb = b.step(ids[0], n, want_logits=True)
+    assert np.array_equal(bits(la), bits(lb))
+    a.prefill(ids)
+    b.prefill(ids)
+    ga, gb = a.generate(1), b.generate(1)       # continues from the panel's prediction
+    assert ga[0] == gb[0] and np.array_equal(bits(ga[1]), bits(gb[1]))
+
+
+def test_panel_infinite_values_stay_with_their_positions(tmpdir_mi):
+    """V rows that overflow fp16 at some positions: tokens before them are untouched (a
+    masked position adds 0 * V, which must not reach a token that does not see it)"""
+    path = synth_cached("panel-hd64", TINY, 31, qk_bias_std=2.0, norm_offset=1.0)
+    with open(path, "rb") as f:
+        data = bytearray(f.read())
+    ty, dims, off = gguf_tensor(path, "blk.1.attn_v.weight")
+    assert ty == 2
+    nb = dims[0] // 32
+    w = np.frombuffer(data, np.uint8, count=nb * 18, offset=off).reshape(nb, 18).copy()
+    w[:, :2] = np.full(nb, 900.0, np.float16).view(np.uint8).reshape(nb, 2)
+    data[off:off + w.size] = w.tobytes()         # row 0 of V: a sum of order 900 * 4.6 * 16 over 256 terms
+    big = tmpdir_mi + "/panel-inf.gguf"
+    with open(big, "wb") as f:
+        f.write(bytes(data))
+    n = 150
+    ids = minfer.prompt_ids(3, n, TINY["n_vocab"])
+    a, b = minfer.Engine(big, max_ctx=256), minfer.Engine(big, max_ctx=256, tchunk=7)
+    pa, ma = a.teacher(ids)
+    pb, mb = b.teacher(ids)
+    ma, mb = np.float32(ma), np.float32(mb)
+    a.close()
+    b.close()
+    fin = np.isfinite(mb)
+    print("[gpu-panel] finite margins", int(fin.sum()), "of", n, flush=True)
+    assert 2 <= fin.sum() < n                    # the case has both kinds
+    assert np.array_equal(fin, np.isfinite(ma)) and np.array_equal(bits(ma[fin]), bits(mb[fin])) and pa == pb
