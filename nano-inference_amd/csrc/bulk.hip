@@ -9,7 +9,7 @@
 // Every value equals the single-token step's bit for bit (the reduction plan at the top of
 // kernels.hip):
 //   q4_0 x int8   the integer block dots on int8 MFMA (exact); dw*dx of a block is an outer
-//                 product, taken by an f32 MFMA of depth 1 (exact: 11 x 11 bits); the fp32
+//                 product of fp16 values, taken by an f16 MFMA (exact: 11 x 11 bits); the fp32
 //                 chain acc = fma(dw*dx, float(dot), acc) stays on the VALU. Chunk sums and
 //                 segments are added left to right as everywhere.
 //   attention     an f32 MFMA is a chain of fused multiply-adds in k order (one rounding per
@@ -26,11 +26,13 @@ namespace mi {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x32 __attribute__((ext_vector_type(32)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kBMaxE = kMaxE;
 constexpr int kBThreads = 256;
+constexpr int kKW = 8, kGThreads = 64 * kKW;   // waves of a GEMM workgroup: the chunks it runs at once
 
 // element offset of (token t, block b, element e of the block) in an operand buffer
 __host__ __device__ __forceinline__ size_t bx_at(int nb, int t, int b, int e) {
@@ -53,14 +55,16 @@ BulkSizes bulk_sizes(int E, int FF, int NH, int HD, int QKV, int V, int maxseq, 
     return s;
 }
 
+__device__ __forceinline__ uint16_t f2h_bits(float v) { return __half_as_ushort(__float2half(v)); }
+
 // ------------------------------------------------------------------ GEMM
 // D layout of a 32x32 MFMA tile: lane l holds column l % 32, rows 8(j/4) + 4(l/32) + j%4.
 __device__ __forceinline__ int drow(int j, int half) { return 8 * (j >> 2) + 4 * half + (j & 3); }
 
 // 16 nibbles of one half block as int8 16*(n - 8): the low nibbles (elements 0..15) on
 // lanes 0..31, the high ones (16..31) on lanes 32..63. In the byte's upper half and with
-// its top bit flipped a nibble is the signed byte 16(n - 8); the factor 16 comes off with
-// the scale (a power of two, so exactly).
+// its top bit flipped a nibble is the signed byte 16(n - 8); the factor 16 comes off
+// the finished sums (a power of two, so exactly).
 __device__ __forceinline__ i32x4 unpack16(uint4 w, int sh) {
     const uint32_t m = 0xF0F0F0F0u, x = 0x80808080u;
     return i32x4{(int)(((w.x << sh) & m) ^ x), (int)(((w.y << sh) & m) ^ x), (int)(((w.z << sh) & m) ^ x),
@@ -71,24 +75,26 @@ enum BEpi { BE_PART, BE_RES, BE_GU, BE_LM };
 
 struct BStage {                    // one pair of blocks: 64 weight rows, 64 tokens
     uint4 a[2][2];                 // [32-row tile][block]
-    uint4 b[2][2];                 // [32-token tile][block]
-    float dx[2];                   // token scales: block 2p on lanes 0..31, 2p + 1 on 32..63
+    i32x4 b[2][2];                 // [32-token tile][block]
+    uint32_t dx[2];                // token scales (fp16 bits): block 2p on lanes 0..31, 2p + 1 on 32..63
     uint32_t sw[2];                // row scales of both blocks (fp16 x 2), [32-row tile]
 };
 
-// One workgroup: 64 rows x 64 tokens. Wave w takes chunks w, w + 4, ... of the K range: per
-// chunk the 2 x 2 tiles of 32 x 32 outputs run their block chains; then the four waves' chunk
-// sums meet in LDS and wave w adds tile w's in chunk order. Weights and activations go
-// straight to registers (each wave reads its own K range, so there is nothing to share
-// inside the workgroup), one block pair ahead.
+// One workgroup: 64 rows x 64 tokens, eight waves. Wave w takes chunks w, w + 8, ... of the K
+// range: per chunk the 2 x 2 tiles of 32 x 32 outputs run their block chains; then the
+// waves' chunk sums meet in LDS and are added in chunk order, each wave for an eighth of the
+// outputs (both row tiles, token tile w % 2, rows 8(w/2) + 4(l/32) .. + 3). Weights and
+// activations go straight to registers (each wave reads its own K range, so there is nothing
+// to share inside the workgroup), one block pair ahead.
 // W: rows of the GEMM; xq/xd: the first token tile; out[..]: token 0 of the first tile.
 // Grid (1-D): XCD x = id % 8 holds row groups g % 8 == x and walks their token tiles next
 // to each other, so a group's weights come from HBM once and are then in that XCD's L2.
 template <int CB, int EPI>
-__global__ __launch_bounds__(kBThreads, 2) void k_bgemm(PMat W, const int8_t* xq, const float* xd, int ntt, int nseg,
-                                                        float* out, int8_t* oq, float4* cand, int ostride) {
-    __shared__ float4 red[4][4][4][64], totl[4][4][64];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, half = lane >> 5, col = lane & 31;
+__global__ __launch_bounds__(kGThreads, 2) void k_bgemm(PMat W, const int8_t* xq, const uint16_t* xd, int ntt, int nseg,
+                                                        float* out, int8_t* oq, uint16_t* od, float4* cand, int ostride) {
+    __shared__ float4 red[kKW][4][4][64];                    // [chunk of the window][tile][j][lane]
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, half = lane >> 5,
+              col = lane & 31;
     const int ng = W.rows >> 6, per = ntt * nseg, id = blockIdx.x;
     const int k0 = id >> 3, gi = k0 / per, rest = k0 - gi * per, g = gi * 8 + (id & 7);
     if (g >= ng) return;
@@ -97,69 +103,79 @@ __global__ __launch_bounds__(kBThreads, 2) void k_bgemm(PMat W, const int8_t* xq
     const int s0 = nseg > 1 ? sidx : 0, s1 = nseg > 1 ? sidx + 1 : W.ks;
     const int cbeg = s0 * W.nc / W.ks, cend = s1 * W.nc / W.ks;
     const uint8_t* wbase = W.base + (size_t)g * W.nc * (CB * 1152);
-    const int8_t* xt = xq + (size_t)(2 * tt) * W.nb * 1024 + lane * 16;
-    const float* dt = xd + (size_t)(2 * tt) * W.nb * 32 + lane;
+    const int8_t* xt = xq + (size_t)(2 * tt) * W.nb * 1024;
+    const uint16_t* dt = xd + (size_t)(2 * tt) * W.nb * 32;
     const size_t xstep = (size_t)W.nb * 1024, dstep = (size_t)W.nb * 32;
     const int sh = half ? 0 : 4;
 
-    i32x16 magic;                  // float(1.5 * 2^23 + i) has the bits of 0x4B400000 + i, |i| < 2^22
-#pragma unroll
-    for (int j = 0; j < 16; j++) magic[j] = 0x4B400000;
-    asm volatile("" : "+v"(magic));
-
+    // uniform base (the wave's chunk) + lane offset
+    const int woff = col * 16, xoff = lane * 16, soff = CB * 1024 + col * (CB * 2);
     auto load_pair = [&](BStage& s, int c, int p) {
-        const uint8_t* t = wbase + (size_t)c * (CB * 1152) + (2 * p) * 1024 + col * 16;
+        const uint8_t* t = wbase + (size_t)c * (CB * 1152);
         const int b = c * CB + 2 * p;
+        const int8_t* x0 = xt + (size_t)b * 1024;
+        const uint16_t* f0 = dt + (size_t)b * 32;
 #pragma unroll
         for (int k = 0; k < 2; k++) {
-            s.a[0][k] = *reinterpret_cast<const uint4*>(t + k * 1024);
-            s.a[1][k] = *reinterpret_cast<const uint4*>(t + k * 1024 + 512);
-            s.b[0][k] = *reinterpret_cast<const uint4*>(xt + (size_t)(b + k) * 1024);
-            s.b[1][k] = *reinterpret_cast<const uint4*>(xt + xstep + (size_t)(b + k) * 1024);
+            s.a[0][k] = *reinterpret_cast<const uint4*>(t + (2 * p + k) * 1024 + woff);
+            s.a[1][k] = *reinterpret_cast<const uint4*>(t + (2 * p + k) * 1024 + 512 + woff);
+            s.b[0][k] = *reinterpret_cast<const i32x4*>(x0 + k * 1024 + xoff);
+            s.b[1][k] = *reinterpret_cast<const i32x4*>(x0 + xstep + k * 1024 + xoff);
         }
-        s.dx[0] = dt[(size_t)b * 32];
-        s.dx[1] = dt[dstep + (size_t)b * 32];
-        const uint8_t* ts = wbase + (size_t)c * (CB * 1152) + CB * 1024 + col * (CB * 2) + 4 * p;
-        s.sw[0] = *reinterpret_cast<const uint32_t*>(ts);
-        s.sw[1] = *reinterpret_cast<const uint32_t*>(ts + 32 * CB * 2);
+        s.dx[0] = f0[lane];
+        s.dx[1] = (f0 + dstep)[lane];
+        s.sw[0] = *reinterpret_cast<const uint32_t*>(t + 4 * p + soff);
+        s.sw[1] = *reinterpret_cast<const uint32_t*>(t + 4 * p + 32 * CB * 2 + soff);
+        asm volatile("" ::: "memory");                       // issued here, not where they are used
     };
-    f32x16 acc[2][2];
+    float acc[2][2][16];
     auto pair = [&](const BStage& s) {
 #pragma unroll
         for (int r = 0; r < 2; r++) {
             const i32x4 a0 = unpack16(s.a[r][0], sh), a1 = unpack16(s.a[r][1], sh);
-            const uint32_t sw = s.sw[r];
-            const float dw = __fmul_rn(half ? h2f_hi(sw) : h2f_lo(sw), 0.0625f);
+            uint2 dw = make_uint2((s.sw[r] >> (half * 16)) & 0xFFFFu, 0u);
 #pragma unroll
             for (int t = 0; t < 2; t++) {
-                float dt_ = s.dx[t];
-                asm volatile("" : "+v"(dt_));
+                // the asm statements keep one tile's products at a time in registers, and its
+                // conversions together ahead of the chain (back to back they would wait on
+                // each other)
+                uint2 dx = make_uint2(s.dx[t], 0u);
+                i32x4 b0 = s.b[t][0], b1 = s.b[t][1];
+                asm volatile("" : "+v"(dx.x), "+v"(b0), "+v"(b1));
+                // dw * dx of both blocks: k = 0 of a two-block f16 outer product (exact in fp32)
                 f32x32 pr = {};
-                pr = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, dt_, pr, 0, 0, 0);
-                uint4 b0 = s.b[t][0], b1 = s.b[t][1];
-                asm volatile("" : "+v"(b0.x), "+v"(b1.x));
-                const i32x16 d0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(
-                    a0, i32x4{(int)b0.x, (int)b0.y, (int)b0.z, (int)b0.w}, magic, 0, 0, 0);
-                const i32x16 d1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(
-                    a1, i32x4{(int)b1.x, (int)b1.y, (int)b1.z, (int)b1.w}, magic, 0, 0, 0);
+                pr = __builtin_amdgcn_mfma_f32_32x32x4f16(__builtin_bit_cast(f16x4, dw), __builtin_bit_cast(f16x4, dx), pr, 0, 0, 0);
+                i32x16 d0 = {}, d1 = {};
+                d0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, b0, d0, 0, 0, 0);
+                d1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b1, d1, 0, 0, 0);
+                asm volatile("" : "+v"(d0), "+v"(d1), "+v"(pr));
+                f32x16 t0, t1;
 #pragma unroll
-                for (int j = 0; j < 16; j++)
-                    acc[r][t][j] = __fmaf_rn(pr[j], __fsub_rn(__int_as_float(d0[j]), 12582912.f), acc[r][t][j]);
+                for (int j = 0; j < 16; j++) t0[j] = __int2float_rn(d0[j]);
 #pragma unroll
-                for (int j = 0; j < 16; j++)
-                    acc[r][t][j] = __fmaf_rn(pr[16 + j], __fsub_rn(__int_as_float(d1[j]), 12582912.f), acc[r][t][j]);
-                asm volatile("" : "+v"(acc[r][t]));          // one tile's products at a time in registers
+                for (int j = 0; j < 16; j++) t1[j] = __int2float_rn(d1[j]);
+                asm volatile("" : "+v"(t0), "+v"(t1));
+#pragma unroll
+                for (int j = 0; j < 16; j++) acc[r][t][j] = __fmaf_rn(pr[j], t0[j], acc[r][t][j]);
+#pragma unroll
+                for (int j = 0; j < 16; j++) acc[r][t][j] = __fmaf_rn(pr[16 + j], t1[j], acc[r][t][j]);
+                // element by element: a 16-register tuple here turns half of the v_fmac into
+                // v_fma with all operands in one register bank (2.75 against 1.35 ns)
+#pragma unroll
+                for (int j = 0; j < 16; j += 4)
+                    asm volatile("" : "+v"(acc[r][t][j]), "+v"(acc[r][t][j + 1]), "+v"(acc[r][t][j + 2]), "+v"(acc[r][t][j + 3]));
             }
         }
     };
 
     BStage st[2];
-    float sg[16];
+    const int ot = wave & 1, oj = wave >> 1;                 // this wave's share of the outputs
+    float sg[8], tot[8];
 #pragma unroll
-    for (int j = 0; j < 16; j++) sg[j] = 0.f;
+    for (int i = 0; i < 8; i++) sg[i] = tot[i] = 0.f;
     int s = s0, sb = cbeg, se = (s0 + 1) * W.nc / W.ks;      // the segment the sums are in
     if (cbeg + wave < cend) load_pair(st[0], cbeg + wave, 0);
-    for (int c0 = cbeg; c0 < cend; c0 += 4) {
+    for (int c0 = cbeg; c0 < cend; c0 += kKW) {
         const int c = c0 + wave;
         if (c < cend) {
 #pragma unroll
@@ -172,8 +188,8 @@ __global__ __launch_bounds__(kBThreads, 2) void k_bgemm(PMat W, const int8_t* xq
             for (int p = 0; p < CB / 2; p++) {
                 if (p + 1 < CB / 2) {
                     load_pair(st[(p + 1) & 1], c, p + 1);
-                } else if (c + 4 < cend) {
-                    load_pair(st[(p + 1) & 1], c + 4, 0);
+                } else if (c + kKW < cend) {
+                    load_pair(st[(p + 1) & 1], c + kKW, 0);
                 }
                 pair(st[p & 1]);
             }
@@ -188,28 +204,21 @@ __global__ __launch_bounds__(kBThreads, 2) void k_bgemm(PMat W, const int8_t* xq
         }
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < kKW; i++) {
             const int ci = c0 + i;
             if (ci < cend) {
                 const bool first = ci == sb;
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const float4 v = red[i][wave][j][lane];
-                    sg[4 * j] = first ? v.x : __fadd_rn(sg[4 * j], v.x);
-                    sg[4 * j + 1] = first ? v.y : __fadd_rn(sg[4 * j + 1], v.y);
-                    sg[4 * j + 2] = first ? v.z : __fadd_rn(sg[4 * j + 2], v.z);
-                    sg[4 * j + 3] = first ? v.w : __fadd_rn(sg[4 * j + 3], v.w);
+                for (int r = 0; r < 2; r++) {
+                    const float4 v = red[i][2 * r + ot][oj][lane];
+                    sg[4 * r] = first ? v.x : __fadd_rn(sg[4 * r], v.x);
+                    sg[4 * r + 1] = first ? v.y : __fadd_rn(sg[4 * r + 1], v.y);
+                    sg[4 * r + 2] = first ? v.z : __fadd_rn(sg[4 * r + 2], v.z);
+                    sg[4 * r + 3] = first ? v.w : __fadd_rn(sg[4 * r + 3], v.w);
                 }
                 if (ci + 1 == se) {                          // segment done: segments left to right
 #pragma unroll
-                    for (int j = 0; j < 4; j++) {            // the lane's own slot, in LDS to spare registers
-                        float4 v = make_float4(sg[4 * j], sg[4 * j + 1], sg[4 * j + 2], sg[4 * j + 3]);
-                        if (s > s0) {
-                            const float4 o = totl[wave][j][lane];
-                            v = make_float4(__fadd_rn(o.x, v.x), __fadd_rn(o.y, v.y), __fadd_rn(o.z, v.z), __fadd_rn(o.w, v.w));
-                        }
-                        totl[wave][j][lane] = v;
-                    }
+                    for (int j = 0; j < 8; j++) tot[j] = s == s0 ? sg[j] : __fadd_rn(tot[j], sg[j]);
                     s++;
                     sb = se;
                     se = (s + 1) * W.nc / W.ks;
@@ -219,20 +228,18 @@ __global__ __launch_bounds__(kBThreads, 2) void k_bgemm(PMat W, const int8_t* xq
         __syncthreads();
     }
 
-    float tot[16];
+    // the weight codes were 16(n - 8): 1/16 here is exact, and so is every step before (all
+    // terms are multiples of 2^-48, so the chains never meet a denormal)
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const float4 v = totl[wave][j][lane];
-        tot[4 * j] = v.x; tot[4 * j + 1] = v.y; tot[4 * j + 2] = v.z; tot[4 * j + 3] = v.w;
-    }
-    // wave w holds rows 32(w/2).. of the group, tokens 32(w%2).. of the tile
-    const int rt = wave >> 1, tok = (2 * tt + (wave & 1)) * 32 + col;
+    for (int i = 0; i < 8; i++) tot[i] = __fmul_rn(tot[i], 0.0625f);
+    // tot[4r + i]: row 32r + 8 oj + 4 half + i of the group, token tok
+    const int tok = (2 * tt + ot) * 32 + col;
     if constexpr (EPI == BE_PART || EPI == BE_RES) {
-        float* o = out + (size_t)sidx * ostride + (size_t)tok * W.rows + g * 64 + rt * 32 + 4 * half;
+        float* o = out + (size_t)sidx * ostride + (size_t)tok * W.rows + g * 64 + 8 * oj + 4 * half;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            float4 v = make_float4(tot[4 * j], tot[4 * j + 1], tot[4 * j + 2], tot[4 * j + 3]);
-            float4* q = reinterpret_cast<float4*>(o + 8 * j);
+        for (int r = 0; r < 2; r++) {
+            float4 v = make_float4(tot[4 * r], tot[4 * r + 1], tot[4 * r + 2], tot[4 * r + 3]);
+            float4* q = reinterpret_cast<float4*>(o + 32 * r);
             if constexpr (EPI == BE_RES) {
                 const float4 h = *q;
                 v = make_float4(__fadd_rn(h.x, v.x), __fadd_rn(h.y, v.y), __fadd_rn(h.z, v.z), __fadd_rn(h.w, v.w));
@@ -240,55 +247,44 @@ __global__ __launch_bounds__(kBThreads, 2) void k_bgemm(PMat W, const int8_t* xq
             *q = v;
         }
     } else if constexpr (EPI == BE_GU) {
-        // rows 0..31 of a group are gate rows, 32..63 their up rows: silu(g)*u, then one
-        // int8 block per token
-        if (rt == 1)
+        // rows 0..31 of a group are gate rows, 32..63 their up rows: silu(g)*u, then one int8
+        // block per token, its max over the four waves of the token tile
+        float a[4], mx = 0.f;
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                red[0][wave & 1][j][lane] = make_float4(tot[4 * j], tot[4 * j + 1], tot[4 * j + 2], tot[4 * j + 3]);
-        __syncthreads();
-        if (rt == 0) {
-            float a[16], mx = 0.f;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const float4 u = red[0][wave][j][lane];
-                const float uu[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float v = tot[4 * j + i], e = mi_expf(-v);
-                    a[4 * j + i] = __fmul_rn(__fdiv_rn(v, __fadd_rn(1.0f, e)), uu[i]);
-                    mx = fmaxf(mx, fabsf(a[4 * j + i]));
-                }
-            }
-            float x, y;
-            pair32(mx, x, y);
-            mx = fmaxf(x, y);
-            const float inv = mx > 0.f ? __fdiv_rn(127.f, mx) : 0.f;
-            const int nbo = ng;                              // one block per row group
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                uint32_t w = 0;
-#pragma unroll
-                for (int i = 0; i < 4; i++) w |= (uint32_t)(__float2int_rn(__fmul_rn(a[4 * j + i], inv)) & 0xFF) << (8 * i);
-                *reinterpret_cast<uint32_t*>(oq + bx_at(nbo, tok, g, 8 * j + 4 * half)) = w;
-            }
-            if (half == 0) out[bd_at(nbo, tok, g)] = fp16_round(__fdiv_rn(mx, 127.f));
+        for (int i = 0; i < 4; i++) {
+            const float v = tot[i], e = mi_expf(-v);
+            a[i] = __fmul_rn(__fdiv_rn(v, __fadd_rn(1.0f, e)), tot[4 + i]);
+            mx = fmaxf(mx, fabsf(a[i]));
         }
+        float x, y;
+        pair32(mx, x, y);
+        float* ml = reinterpret_cast<float*>(red);           // [4 waves][2 tiles][32 tokens]
+        if (half == 0) ml[(oj * 2 + ot) * 32 + col] = fmaxf(x, y);
+        __syncthreads();
+        mx = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; j++) mx = fmaxf(mx, ml[(j * 2 + ot) * 32 + col]);
+        const float inv = mx > 0.f ? __fdiv_rn(127.f, mx) : 0.f;
+        uint32_t w = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) w |= (uint32_t)(__float2int_rn(__fmul_rn(a[i], inv)) & 0xFF) << (8 * i);
+        *reinterpret_cast<uint32_t*>(oq + bx_at(ng, tok, g, 8 * oj + 4 * half)) = w;
+        if (oj == 0 && half == 0) od[bd_at(ng, tok, g)] = f2h_bits(__fdiv_rn(mx, 127.f));
     } else {
         Top2 t{-__builtin_inff(), INT_MAX, -__builtin_inff()};
 #pragma unroll
-        for (int j = 0; j < 16; j++) top2_push(t, tot[j], g * 64 + rt * 32 + drow(j, half));
-        const auto rb = __builtin_amdgcn_permlane32_swap(__float_as_uint(t.best), __float_as_uint(t.best), false, false);
-        const auto ri = __builtin_amdgcn_permlane32_swap((unsigned)t.idx, (unsigned)t.idx, false, false);
-        const auto rs = __builtin_amdgcn_permlane32_swap(__float_as_uint(t.second), __float_as_uint(t.second), false, false);
-        Top2 x{__uint_as_float(rb[0]), (int)ri[0], __uint_as_float(rs[0])};
-        top2_merge(x, __uint_as_float(rb[1]), (int)ri[1], __uint_as_float(rs[1]));
-        if (rt == 1) red[0][wave & 1][0][lane] = make_float4(x.best, __int_as_float(x.idx), x.second, 0.f);
+        for (int i = 0; i < 8; i++) top2_push(t, tot[i], g * 64 + 32 * (i >> 2) + 8 * oj + 4 * half + (i & 3));
+        float4* tl = &red[0][0][0][0];                       // [4 waves][2 tiles][64 lanes]
+        tl[(oj * 2 + ot) * 64 + lane] = make_float4(t.best, __int_as_float(t.idx), t.second, 0.f);
         __syncthreads();
-        if (rt == 0 && half == 0) {
-            const float4 o = red[0][wave][0][lane];
-            top2_merge(x, o.x, __float_as_int(o.y), o.z);
-            cand[(size_t)tok * ng + g] = make_float4(x.best, __int_as_float(x.idx), x.second, 0.f);
+        if (oj == 0 && half == 0) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                if (j == 0) continue;
+                const float4 o = tl[((j >> 1) * 2 + ot) * 64 + 32 * (j & 1) + col];
+                top2_merge(t, o.x, __float_as_int(o.y), o.z);
+            }
+            cand[(size_t)tok * ng + g] = make_float4(t.best, __int_as_float(t.idx), t.second, 0.f);
         }
     }
 }
@@ -315,7 +311,7 @@ __global__ __launch_bounds__(64) void k_bargmax(const float4* cand, int ng, int 
 // 256j + 4l .. + 3, the order of the canonical sum of squares (rms_scale).
 __global__ __launch_bounds__(kBThreads) void k_bnorm(int n, float eps, const float* w, float* h, const float* emb,
                                                      const int32_t* tok, const float* part, int ks, int m, int8_t* xq,
-                                                     float* xd) {
+                                                     uint16_t* xd) {
     constexpr int NJ = kBMaxE / 256;
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (t >= m) return;
@@ -364,7 +360,7 @@ __global__ __launch_bounds__(kBThreads) void k_bnorm(int n, float eps, const flo
         if (own) {
             *reinterpret_cast<uint32_t*>(xq + bx_at(nb, t, e >> 5, e & 31)) =
                 (uint32_t)(q0 & 0xFF) | ((uint32_t)(q1 & 0xFF) << 8) | ((uint32_t)(q2 & 0xFF) << 16) | ((uint32_t)q3 << 24);
-            if ((lane & 7) == 0) xd[bd_at(nb, t, e >> 5)] = fp16_round(__fdiv_rn(mx, 127.f));
+            if ((lane & 7) == 0) xd[bd_at(nb, t, e >> 5)] = f2h_bits(__fdiv_rn(mx, 127.f));
         }
     }
 }
@@ -629,7 +625,7 @@ __global__ __launch_bounds__(kBThreads, 1) void k_battn(const float* qkv, int QK
 // the O GEMM's operand
 template <int HD>
 __global__ __launch_bounds__(kBThreads) void k_bcomb(const float* rec, int NH, int m, int p0, int nsp, int nb, int8_t* xq,
-                                                     float* xd) {
+                                                     uint16_t* xd) {
     constexpr int DPL = HD / 64;
     const int item = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (item >= m * NH) return;
@@ -665,17 +661,17 @@ __global__ __launch_bounds__(kBThreads) void k_bcomb(const float* rec, int NH, i
         const uint32_t b = (uint32_t)(q & 0xFF);
         const uint32_t wd = b | (__shfl_down(b, 1) << 8) | (__shfl_down(b, 2) << 16) | (__shfl_down(b, 3) << 24);
         if ((lane & 3) == 0) *reinterpret_cast<uint32_t*>(xq + bx_at(nb, t, el >> 5, el & 31)) = wd;
-        if ((lane & 31) == 0) xd[bd_at(nb, t, el >> 5)] = d;
+        if ((lane & 31) == 0) xd[bd_at(nb, t, el >> 5)] = f2h_bits(d);
     }
 }
 
 // ------------------------------------------------------------------ host side
 template <int EPI>
-static void gemm(const PMat& W, const int8_t* xq, const float* xd, int ntt, int nseg, float* out, int8_t* oq, float4* cand,
-                 int ostride, hipStream_t s) {
+static void gemm(const PMat& W, const int8_t* xq, const uint16_t* xd, int ntt, int nseg, float* out, int8_t* oq,
+                 uint16_t* od, float4* cand, int ostride, hipStream_t s) {
     const int grid = 8 * (((W.rows >> 6) + 7) / 8) * ntt * nseg;
-    if (W.cb == 8) LAUNCH((k_bgemm<8, EPI>), grid, kBThreads, s, W, xq, xd, ntt, nseg, out, oq, cand, ostride);
-    else LAUNCH((k_bgemm<4, EPI>), grid, kBThreads, s, W, xq, xd, ntt, nseg, out, oq, cand, ostride);
+    if (W.cb == 8) LAUNCH((k_bgemm<8, EPI>), grid, kGThreads, s, W, xq, xd, ntt, nseg, out, oq, od, cand, ostride);
+    else LAUNCH((k_bgemm<4, EPI>), grid, kGThreads, s, W, xq, xd, ntt, nseg, out, oq, od, cand, ostride);
 }
 
 void launch_bulk(const DModel& M, const DLayer* layers, const BulkBuf& B, int p0, int m, bool all, bool last,
@@ -689,7 +685,7 @@ void launch_bulk(const DModel& M, const DLayer* layers, const BulkBuf& B, int p0
     for (int l = 0; l < M.NL; l++) {
         const DLayer& L = layers[l];
         norm(L.an, l == 0 ? M.emb : nullptr, ks);
-        gemm<BE_PART>(L.qkv, B.xq, B.xd, ntt, 1, B.qkv, nullptr, nullptr, 0, s);
+        gemm<BE_PART>(L.qkv, B.xq, B.xd, ntt, 1, B.qkv, nullptr, nullptr, nullptr, 0, s);
         const size_t kv = (size_t)l * M.NKV * M.maxseq * M.HD;
         auto attn = [&](auto hd) {
             constexpr int HD = decltype(hd)::value;
@@ -702,18 +698,18 @@ void launch_bulk(const DModel& M, const DLayer* layers, const BulkBuf& B, int p0
         };
         if (M.HD == 64) attn(std::integral_constant<int, 64>());
         else attn(std::integral_constant<int, 128>());
-        gemm<BE_RES>(L.o, B.xq, B.xd, ntt, 1, B.h, nullptr, nullptr, 0, s);
+        gemm<BE_RES>(L.o, B.xq, B.xd, ntt, 1, B.h, nullptr, nullptr, nullptr, 0, s);
         norm(L.fn, nullptr, 0);
-        gemm<BE_GU>(L.gu, B.xq, B.xd, ntt, 1, B.ad, B.aq, nullptr, 0, s);
+        gemm<BE_GU>(L.gu, B.xq, B.xd, ntt, 1, nullptr, B.aq, B.ad, nullptr, 0, s);
         ks = ntt * 64 <= kBulkSplitM ? L.d.ks : 0;
-        if (ks) gemm<BE_PART>(L.d, B.aq, B.ad, ntt, ks, B.dpart, nullptr, nullptr, kBulkSplitM * E, s);
-        else gemm<BE_RES>(L.d, B.aq, B.ad, ntt, 1, B.h, nullptr, nullptr, 0, s);
+        if (ks) gemm<BE_PART>(L.d, B.aq, B.ad, ntt, ks, B.dpart, nullptr, nullptr, nullptr, kBulkSplitM * E, s);
+        else gemm<BE_RES>(L.d, B.aq, B.ad, ntt, 1, B.h, nullptr, nullptr, nullptr, 0, s);
     }
     if (!all && !last) return;
     norm(M.out_norm, nullptr, ks);
     // predictions: every token tile, or only the one that holds the last token
     const int tt0 = all ? 0 : ntt - 1, t0 = all ? 0 : m - 1;
-    gemm<BE_LM>(M.lm, B.xq + (size_t)(2 * tt0) * nbE * 1024, B.xd + (size_t)(2 * tt0) * nbE * 32, ntt - tt0, 1, nullptr, nullptr,
+    gemm<BE_LM>(M.lm, B.xq + (size_t)(2 * tt0) * nbE * 1024, B.xd + (size_t)(2 * tt0) * nbE * 32, ntt - tt0, 1, nullptr, nullptr, nullptr,
                 B.cand + (size_t)tt0 * 64 * (M.V / 64), 0, s);
     LAUNCH(k_bargmax, m - t0, 64, s, B.cand, M.V / 64, M.V, t0, p0, M.out_tok, M.out_margin);
 }
