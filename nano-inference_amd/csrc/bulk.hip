@@ -32,6 +32,7 @@ typedef int i32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kBMaxE = kMaxE;
 constexpr int kBThreads = 256;
+constexpr int kBulkWgs = 288;      // 9/8 of the 256 CUs
 constexpr int kKW = 8, kGThreads = 64 * kKW;   // waves of a GEMM workgroup: the chunks it runs at once
 
 // element offset of (token t, block b, element e of the block) in an operand buffer
@@ -65,13 +66,70 @@ __device__ __forceinline__ int drow(int j, int half) { return 8 * (j >> 2) + 4 *
 // lanes 0..31, the high ones (16..31) on lanes 32..63. In the byte's upper half and with
 // its top bit flipped a nibble is the signed byte 16(n - 8); the factor 16 comes off
 // the finished sums (a power of two, so exactly).
-__device__ __forceinline__ i32x4 unpack16(uint4 w, int sh) {
+template <class V>
+__device__ __forceinline__ i32x4 unpack16(V w, int sh) {
     const uint32_t m = 0xF0F0F0F0u, x = 0x80808080u;
-    return i32x4{(int)(((w.x << sh) & m) ^ x), (int)(((w.y << sh) & m) ^ x), (int)(((w.z << sh) & m) ^ x),
-                 (int)(((w.w << sh) & m) ^ x)};
+    return i32x4{(int)((((uint32_t)w.x << sh) & m) ^ x), (int)((((uint32_t)w.y << sh) & m) ^ x),
+                 (int)((((uint32_t)w.z << sh) & m) ^ x), (int)((((uint32_t)w.w << sh) & m) ^ x)};
 }
 
 enum BEpi { BE_PART, BE_RES, BE_GU, BE_LM };
+
+// One 32 x 32 tile, two blocks: acc += their terms of the chain. a0, a1: the blocks' weight
+// codes (unpack16); b0, b1: the tokens' codes; dw, dx: fp16 bits of the row and token scales,
+// the first block's on lanes 0..31, the second's on 32..63.
+// The asm statements keep one tile's products at a time in registers, and its conversions
+// together ahead of the chain (back to back they would wait on each other). 109 ns per SIMD
+// with two waves on it, of which the 64 vector instructions are 97; with the outer product
+// on the f32 MFMA 136, on the vector unit 113, with f16 dots (no conversion) 109-115.
+__device__ __forceinline__ void tile_pair(float (&acc)[16], i32x4 a0, i32x4 a1, i32x4 b0, i32x4 b1, uint32_t dw, uint32_t dx) {
+    uint2 dw2 = make_uint2(dw, 0u), dx2 = make_uint2(dx, 0u);
+    asm volatile("" : "+v"(dx2.x), "+v"(b0), "+v"(b1));
+    // dw * dx of both blocks: k = 0 of a two-block f16 outer product (exact in fp32)
+    f32x32 pr = {};
+    pr = __builtin_amdgcn_mfma_f32_32x32x4f16(__builtin_bit_cast(f16x4, dw2), __builtin_bit_cast(f16x4, dx2), pr, 0, 0, 0);
+    i32x16 d0 = {}, d1 = {};
+    d0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, b0, d0, 0, 0, 0);
+    d1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b1, d1, 0, 0, 0);
+    asm volatile("" : "+v"(d0), "+v"(d1), "+v"(pr));
+    f32x16 t0, t1;
+#pragma unroll
+    for (int j = 0; j < 16; j++) t0[j] = __int2float_rn(d0[j]);
+#pragma unroll
+    for (int j = 0; j < 16; j++) t1[j] = __int2float_rn(d1[j]);
+    asm volatile("" : "+v"(t0), "+v"(t1));
+#pragma unroll
+    for (int j = 0; j < 16; j++) acc[j] = __fmaf_rn(pr[j], t0[j], acc[j]);
+#pragma unroll
+    for (int j = 0; j < 16; j++) acc[j] = __fmaf_rn(pr[16 + j], t1[j], acc[j]);
+    // element by element: a 16-register tuple here turns half of the v_fmac into v_fma with
+    // all operands in one register bank (2.75 against 1.35 ns)
+#pragma unroll
+    for (int j = 0; j < 16; j += 4) asm volatile("" : "+v"(acc[j]), "+v"(acc[j + 1]), "+v"(acc[j + 2]), "+v"(acc[j + 3]));
+}
+
+// gate and up sums of the same 16 rows (D layout) and token: silu(g)*u, then the token's int8
+// block, codes packed per 4 rows; returns the block scale
+__device__ __forceinline__ float silu_quant(const float (&gt)[16], const float (&up)[16], uint32_t (&w)[4]) {
+    float a[16], mx = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const float e = mi_expf(-gt[i]);
+        a[i] = __fmul_rn(__fdiv_rn(gt[i], __fadd_rn(1.0f, e)), up[i]);
+        mx = fmaxf(mx, fabsf(a[i]));
+    }
+    float x, y;
+    pair32(mx, x, y);
+    mx = fmaxf(x, y);
+    const float inv = mx > 0.f ? __fdiv_rn(127.f, mx) : 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        w[j] = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) w[j] |= (uint32_t)(__float2int_rn(__fmul_rn(a[4 * j + i], inv)) & 0xFF) << (8 * i);
+    }
+    return __fdiv_rn(mx, 127.f);
+}
 
 struct BStage {                    // one pair of blocks: 64 weight rows, 64 tokens
     uint4 a[2][2];                 // [32-row tile][block]
@@ -90,8 +148,8 @@ struct BStage {                    // one pair of blocks: 64 weight rows, 64 tok
 // Grid (1-D): XCD x = id % 8 holds row groups g % 8 == x and walks their token tiles next
 // to each other, so a group's weights come from HBM once and are then in that XCD's L2.
 template <int CB, int EPI>
-__global__ __launch_bounds__(kGThreads, 2) void k_bgemm(PMat W, const int8_t* xq, const uint16_t* xd, int ntt, int nseg,
-                                                        float* out, int8_t* oq, uint16_t* od, float4* cand, int ostride) {
+__global__ __launch_bounds__(kGThreads, 2) void k_bgemm(PMat W, const int8_t* xq, const uint32_t* xd, int ntt, int nseg,
+                                                        float* out, int ostride, int8_t* oq, uint32_t* od) {
     __shared__ float4 red[kKW][4][4][64];                    // [chunk of the window][tile][j][lane]
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, half = lane >> 5,
               col = lane & 31;
@@ -104,7 +162,7 @@ __global__ __launch_bounds__(kGThreads, 2) void k_bgemm(PMat W, const int8_t* xq
     const int cbeg = s0 * W.nc / W.ks, cend = s1 * W.nc / W.ks;
     const uint8_t* wbase = W.base + (size_t)g * W.nc * (CB * 1152);
     const int8_t* xt = xq + (size_t)(2 * tt) * W.nb * 1024;
-    const uint16_t* dt = xd + (size_t)(2 * tt) * W.nb * 32;
+    const uint32_t* dt = xd + (size_t)(2 * tt) * W.nb * 32;
     const size_t xstep = (size_t)W.nb * 1024, dstep = (size_t)W.nb * 32;
     const int sh = half ? 0 : 4;
 
@@ -114,7 +172,7 @@ __global__ __launch_bounds__(kGThreads, 2) void k_bgemm(PMat W, const int8_t* xq
         const uint8_t* t = wbase + (size_t)c * (CB * 1152);
         const int b = c * CB + 2 * p;
         const int8_t* x0 = xt + (size_t)b * 1024;
-        const uint16_t* f0 = dt + (size_t)b * 32;
+        const uint32_t* f0 = dt + (size_t)b * 32;
 #pragma unroll
         for (int k = 0; k < 2; k++) {
             s.a[0][k] = *reinterpret_cast<const uint4*>(t + (2 * p + k) * 1024 + woff);
@@ -133,38 +191,9 @@ __global__ __launch_bounds__(kGThreads, 2) void k_bgemm(PMat W, const int8_t* xq
 #pragma unroll
         for (int r = 0; r < 2; r++) {
             const i32x4 a0 = unpack16(s.a[r][0], sh), a1 = unpack16(s.a[r][1], sh);
-            uint2 dw = make_uint2((s.sw[r] >> (half * 16)) & 0xFFFFu, 0u);
+            const uint32_t dw = (s.sw[r] >> (half * 16)) & 0xFFFFu;
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
-                // the asm statements keep one tile's products at a time in registers, and its
-                // conversions together ahead of the chain (back to back they would wait on
-                // each other)
-                uint2 dx = make_uint2(s.dx[t], 0u);
-                i32x4 b0 = s.b[t][0], b1 = s.b[t][1];
-                asm volatile("" : "+v"(dx.x), "+v"(b0), "+v"(b1));
-                // dw * dx of both blocks: k = 0 of a two-block f16 outer product (exact in fp32)
-                f32x32 pr = {};
-                pr = __builtin_amdgcn_mfma_f32_32x32x4f16(__builtin_bit_cast(f16x4, dw), __builtin_bit_cast(f16x4, dx), pr, 0, 0, 0);
-                i32x16 d0 = {}, d1 = {};
-                d0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, b0, d0, 0, 0, 0);
-                d1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b1, d1, 0, 0, 0);
-                asm volatile("" : "+v"(d0), "+v"(d1), "+v"(pr));
-                f32x16 t0, t1;
-#pragma unroll
-                for (int j = 0; j < 16; j++) t0[j] = __int2float_rn(d0[j]);
-#pragma unroll
-                for (int j = 0; j < 16; j++) t1[j] = __int2float_rn(d1[j]);
-                asm volatile("" : "+v"(t0), "+v"(t1));
-#pragma unroll
-                for (int j = 0; j < 16; j++) acc[r][t][j] = __fmaf_rn(pr[j], t0[j], acc[r][t][j]);
-#pragma unroll
-                for (int j = 0; j < 16; j++) acc[r][t][j] = __fmaf_rn(pr[16 + j], t1[j], acc[r][t][j]);
-                // element by element: a 16-register tuple here turns half of the v_fmac into
-                // v_fma with all operands in one register bank (2.75 against 1.35 ns)
-#pragma unroll
-                for (int j = 0; j < 16; j += 4)
-                    asm volatile("" : "+v"(acc[r][t][j]), "+v"(acc[r][t][j + 1]), "+v"(acc[r][t][j + 2]), "+v"(acc[r][t][j + 3]));
-            }
+            for (int t = 0; t < 2; t++) tile_pair(acc[r][t], a0, a1, s.b[t][0], s.b[t][1], dw, s.dx[t]);
         }
     };
 
@@ -234,7 +263,7 @@ __global__ __launch_bounds__(kGThreads, 2) void k_bgemm(PMat W, const int8_t* xq
     for (int i = 0; i < 8; i++) tot[i] = __fmul_rn(tot[i], 0.0625f);
     // tot[4r + i]: row 32r + 8 oj + 4 half + i of the group, token tok
     const int tok = (2 * tt + ot) * 32 + col;
-    if constexpr (EPI == BE_PART || EPI == BE_RES) {
+    if constexpr (EPI != BE_GU) {
         float* o = out + (size_t)sidx * ostride + (size_t)tok * W.rows + g * 64 + 8 * oj + 4 * half;
 #pragma unroll
         for (int r = 0; r < 2; r++) {
@@ -246,14 +275,14 @@ __global__ __launch_bounds__(kGThreads, 2) void k_bgemm(PMat W, const int8_t* xq
             }
             *q = v;
         }
-    } else if constexpr (EPI == BE_GU) {
+    } else {
         // rows 0..31 of a group are gate rows, 32..63 their up rows: silu(g)*u, then one int8
         // block per token, its max over the four waves of the token tile
         float a[4], mx = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const float v = tot[i], e = mi_expf(-v);
-            a[i] = __fmul_rn(__fdiv_rn(v, __fadd_rn(1.0f, e)), tot[4 + i]);
+            const float e = mi_expf(-tot[i]);
+            a[i] = __fmul_rn(__fdiv_rn(tot[i], __fadd_rn(1.0f, e)), tot[4 + i]);
             mx = fmaxf(mx, fabsf(a[i]));
         }
         float x, y;
@@ -270,22 +299,158 @@ __global__ __launch_bounds__(kGThreads, 2) void k_bgemm(PMat W, const int8_t* xq
         for (int i = 0; i < 4; i++) w |= (uint32_t)(__float2int_rn(__fmul_rn(a[i], inv)) & 0xFF) << (8 * i);
         *reinterpret_cast<uint32_t*>(oq + bx_at(ng, tok, g, 8 * oj + 4 * half)) = w;
         if (oj == 0 && half == 0) od[bd_at(ng, tok, g)] = f2h_bits(__fdiv_rn(mx, 127.f));
-    } else {
-        Top2 t{-__builtin_inff(), INT_MAX, -__builtin_inff()};
+    }
+}
+
+// The same product for gate/up and lm_head, whose row groups alone fill the chip: no K split
+// (their plan has one segment), so no exchange of chunk sums; each wave runs 32 rows x 64
+// tokens through all of K and keeps the running sums in registers. A workgroup is 64 rows x
+// 128 tokens, two workgroups per CU. Weights and activations are loaded four block pairs
+// ahead: a wave's loads return in order, so the activations (L2) wait for the weights (HBM)
+// issued before them.
+// GU: the group's gate rows 0..31 and up rows 32..63 meet in LDS, silu(g)*u -> oq / od.
+// LM: the group's argmax candidate per token -> cand.
+template <int CB, int EPI>
+__global__ __launch_bounds__(kBThreads, 2) void k_bgemm_w(PMat W, const int8_t* xq, const uint32_t* xd, int ntt, int8_t* oq,
+                                                          uint32_t* od, float4* cand) {
+    __shared__ float4 ex[4][2][4][64];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, half = lane >> 5,
+              col = lane & 31;
+    const int ng = W.rows >> 6, per = (ntt + 1) >> 1, id = blockIdx.x;
+    const int k0 = id >> 3, gi = k0 / per, g = gi * 8 + (id & 7);
+    if (g >= ng) return;
+    const int rt = wave & 1, tt = 2 * (k0 - gi * per) + (wave >> 1);
+    const bool active = tt < ntt;                            // an odd number of token tiles
+    constexpr int PC = CB / 2;                               // block pairs per chunk
+    const int np = W.nb / 2, sh = half ? 0 : 4;
+    const uint8_t* wb = W.base + (size_t)g * W.nc * (CB * 1152) + rt * 512;
+    const uint8_t* wsc = W.base + (size_t)g * W.nc * (CB * 1152) + CB * 1024 + rt * 32 * CB * 2;
+    const int8_t* x0 = xq + (size_t)(2 * tt) * W.nb * 1024;
+    const uint32_t* f0 = xd + (size_t)(2 * tt) * W.nb * 32;
+    const size_t xstep = (size_t)W.nb * 1024, dstep = (size_t)W.nb * 32;
+    const int woff = col * 16, xoff = lane * 16, soff = col * (CB * 2);
+
+    struct Slot { i32x4 a[2], b[2][2]; uint32_t sw, dx[2]; };
+    auto load = [&](Slot& s, int q) {
+        const int c = q / PC, p = q - c * PC;
+        const uint8_t* t = wb + (size_t)c * (CB * 1152) + 2 * p * 1024;
+        const int8_t* x = x0 + (size_t)q * 2048;
+        const uint32_t* f = f0 + (size_t)q * 64;
+        s.sw = *reinterpret_cast<const uint32_t*>(wsc + (size_t)c * (CB * 1152) + 4 * p + soff);
+        s.dx[0] = f[lane];
+        s.dx[1] = (f + dstep)[lane];
 #pragma unroll
-        for (int i = 0; i < 8; i++) top2_push(t, tot[i], g * 64 + 32 * (i >> 2) + 8 * oj + 4 * half + (i & 3));
-        float4* tl = &red[0][0][0][0];                       // [4 waves][2 tiles][64 lanes]
-        tl[(oj * 2 + ot) * 64 + lane] = make_float4(t.best, __int_as_float(t.idx), t.second, 0.f);
-        __syncthreads();
-        if (oj == 0 && half == 0) {
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                if (j == 0) continue;
-                const float4 o = tl[((j >> 1) * 2 + ot) * 64 + 32 * (j & 1) + col];
-                top2_merge(t, o.x, __float_as_int(o.y), o.z);
-            }
-            cand[(size_t)tok * ng + g] = make_float4(t.best, __int_as_float(t.idx), t.second, 0.f);
+        for (int k = 0; k < 2; k++) {
+            s.a[k] = *reinterpret_cast<const i32x4*>(t + k * 1024 + woff);
+            s.b[0][k] = *reinterpret_cast<const i32x4*>(x + k * 1024 + xoff);
+            s.b[1][k] = *reinterpret_cast<const i32x4*>(x + xstep + k * 1024 + xoff);
         }
+        asm volatile("" ::: "memory");                       // issued here, not where they are used
+    };
+    constexpr int NS = 4;
+    Slot sl[NS];
+    float acc[2][16];
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int j = 0; j < 16; j++) acc[t][j] = 0.f;
+    // the running sums, each lane's own words in LDS (in registers they would make the loop
+    // spill, and a reload waits for every load in flight); -0 + x = x
+    float4 (&sum)[2][4][64] = ex[wave];
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) sum[t][j][lane] = make_float4(-0.f, -0.f, -0.f, -0.f);
+    if (active) {
+        // past the end the last pair is loaded again (a branch around the load keeps the old
+        // slot alive and costs copies)
+#pragma unroll
+        for (int u = 0; u < NS; u++) load(sl[u], min(u, np - 1));
+        auto step = [&](Slot& s, int q, bool chunk_end) {
+            // nothing of this pair is computed (and so waited for) before the last one is done
+            asm volatile("" : "+v"(s.sw), "+v"(s.a[0]), "+v"(s.a[1]));
+            const i32x4 a0 = unpack16(s.a[0], sh), a1 = unpack16(s.a[1], sh);
+            const uint32_t dw = (s.sw >> (half * 16)) & 0xFFFFu;
+#pragma unroll
+            for (int t = 0; t < 2; t++) tile_pair(acc[t], a0, a1, s.b[t][0], s.b[t][1], dw, s.dx[t]);
+            load(s, min(q + NS, np - 1));
+            if (chunk_end) {                                 // compile time: a chunk is 2 or 4 pairs
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const float4 v = sum[t][j][lane];
+                        sum[t][j][lane] = make_float4(__fadd_rn(v.x, acc[t][4 * j]), __fadd_rn(v.y, acc[t][4 * j + 1]),
+                                                      __fadd_rn(v.z, acc[t][4 * j + 2]), __fadd_rn(v.w, acc[t][4 * j + 3]));
+                        acc[t][4 * j] = acc[t][4 * j + 1] = acc[t][4 * j + 2] = acc[t][4 * j + 3] = 0.f;
+                    }
+            }
+        };
+        // no branch inside the four steps: the compiler then counts the loads in flight exactly
+        int q = 0;
+        for (; q + NS <= np; q += NS)
+#pragma unroll
+            for (int u = 0; u < NS; u++) step(sl[u], q + u, (u + 1) % PC == 0);
+        if constexpr (CB == 4)
+            if (q < np) {                                    // an odd number of chunks of two pairs
+                step(sl[0], q, false);
+                step(sl[1], q + 1, true);
+            }
+    }
+    // 1/16: the weight codes were 16(n - 8)
+    float sg[2][16];
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float4 v = sum[t][j][lane];
+            sg[t][4 * j] = __fmul_rn(v.x, 0.0625f); sg[t][4 * j + 1] = __fmul_rn(v.y, 0.0625f);
+            sg[t][4 * j + 2] = __fmul_rn(v.z, 0.0625f); sg[t][4 * j + 3] = __fmul_rn(v.w, 0.0625f);
+        }
+    if constexpr (EPI == BE_GU) {
+        // wave rt finishes token tile rt of its pair: it hands the other one over
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            ex[wave][0][j][lane] = rt ? make_float4(sg[0][4 * j], sg[0][4 * j + 1], sg[0][4 * j + 2], sg[0][4 * j + 3])
+                                   : make_float4(sg[1][4 * j], sg[1][4 * j + 1], sg[1][4 * j + 2], sg[1][4 * j + 3]);
+        __syncthreads();
+        if (!active) return;
+        float gt[16], up[16];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float4 o = ex[wave ^ 1][0][j][lane];
+            const float ov[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                gt[4 * j + i] = rt ? ov[i] : sg[0][4 * j + i];
+                up[4 * j + i] = rt ? sg[1][4 * j + i] : ov[i];
+            }
+        }
+        const int tok = (2 * tt + rt) * 32 + col;
+        uint32_t w[4];
+        const float d = silu_quant(gt, up, w);
+#pragma unroll
+        for (int j = 0; j < 4; j++) *reinterpret_cast<uint32_t*>(oq + bx_at(ng, tok, g, 8 * j + 4 * half)) = w[j];
+        if (half == 0) od[bd_at(ng, tok, g)] = f2h_bits(d);
+    } else {
+        Top2 tp[2];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            tp[t] = Top2{-__builtin_inff(), INT_MAX, -__builtin_inff()};
+#pragma unroll
+            for (int j = 0; j < 16; j++) top2_push(tp[t], sg[t][j], g * 64 + rt * 32 + drow(j, half));
+            ex[wave][0][t][lane] = make_float4(tp[t].best, __int_as_float(tp[t].idx), tp[t].second, 0.f);
+        }
+        __syncthreads();
+        if (!active || half) return;
+        // wave rt: token tile rt; the four parts are its two halves and the other wave's
+        Top2 a{-__builtin_inff(), INT_MAX, -__builtin_inff()};
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const float4 o = ex[(wave & 2) + (k >> 1)][0][rt][32 * (k & 1) + col];
+            top2_merge(a, o.x, __float_as_int(o.y), o.z);
+        }
+        cand[(size_t)((2 * tt + rt) * 32 + col) * ng + g] = make_float4(a.best, __int_as_float(a.idx), a.second, 0.f);
     }
 }
 
@@ -311,7 +476,7 @@ __global__ __launch_bounds__(64) void k_bargmax(const float4* cand, int ng, int 
 // 256j + 4l .. + 3, the order of the canonical sum of squares (rms_scale).
 __global__ __launch_bounds__(kBThreads) void k_bnorm(int n, float eps, const float* w, float* h, const float* emb,
                                                      const int32_t* tok, const float* part, int ks, int m, int8_t* xq,
-                                                     uint16_t* xd) {
+                                                     uint32_t* xd) {
     constexpr int NJ = kBMaxE / 256;
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (t >= m) return;
@@ -625,7 +790,7 @@ __global__ __launch_bounds__(kBThreads, 1) void k_battn(const float* qkv, int QK
 // the O GEMM's operand
 template <int HD>
 __global__ __launch_bounds__(kBThreads) void k_bcomb(const float* rec, int NH, int m, int p0, int nsp, int nb, int8_t* xq,
-                                                     uint16_t* xd) {
+                                                     uint32_t* xd) {
     constexpr int DPL = HD / 64;
     const int item = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (item >= m * NH) return;
@@ -667,11 +832,18 @@ __global__ __launch_bounds__(kBThreads) void k_bcomb(const float* rec, int NH, i
 
 // ------------------------------------------------------------------ host side
 template <int EPI>
-static void gemm(const PMat& W, const int8_t* xq, const uint16_t* xd, int ntt, int nseg, float* out, int8_t* oq,
-                 uint16_t* od, float4* cand, int ostride, hipStream_t s) {
+static void gemm(const PMat& W, const int8_t* xq, const uint32_t* xd, int ntt, int nseg, float* out, int ostride, int8_t* oq,
+                 uint32_t* od, hipStream_t s) {
     const int grid = 8 * (((W.rows >> 6) + 7) / 8) * ntt * nseg;
-    if (W.cb == 8) LAUNCH((k_bgemm<8, EPI>), grid, kGThreads, s, W, xq, xd, ntt, nseg, out, oq, od, cand, ostride);
-    else LAUNCH((k_bgemm<4, EPI>), grid, kGThreads, s, W, xq, xd, ntt, nseg, out, oq, od, cand, ostride);
+    if (W.cb == 8) LAUNCH((k_bgemm<8, EPI>), grid, kGThreads, s, W, xq, xd, ntt, nseg, out, ostride, oq, od);
+    else LAUNCH((k_bgemm<4, EPI>), grid, kGThreads, s, W, xq, xd, ntt, nseg, out, ostride, oq, od);
+}
+template <int EPI>
+static void gemm_w(const PMat& W, const int8_t* xq, const uint32_t* xd, int ntt, int8_t* oq, uint32_t* od, float4* cand,
+                   hipStream_t s) {
+    const int grid = 8 * (((W.rows >> 6) + 7) / 8) * ((ntt + 1) / 2);
+    if (W.cb == 8) LAUNCH((k_bgemm_w<8, EPI>), grid, kBThreads, s, W, xq, xd, ntt, oq, od, cand);
+    else LAUNCH((k_bgemm_w<4, EPI>), grid, kBThreads, s, W, xq, xd, ntt, oq, od, cand);
 }
 
 void launch_bulk(const DModel& M, const DLayer* layers, const BulkBuf& B, int p0, int m, bool all, bool last,
@@ -685,7 +857,7 @@ void launch_bulk(const DModel& M, const DLayer* layers, const BulkBuf& B, int p0
     for (int l = 0; l < M.NL; l++) {
         const DLayer& L = layers[l];
         norm(L.an, l == 0 ? M.emb : nullptr, ks);
-        gemm<BE_PART>(L.qkv, B.xq, B.xd, ntt, 1, B.qkv, nullptr, nullptr, nullptr, 0, s);
+        gemm<BE_PART>(L.qkv, B.xq, B.xd, ntt, 1, B.qkv, 0, nullptr, nullptr, s);
         const size_t kv = (size_t)l * M.NKV * M.maxseq * M.HD;
         auto attn = [&](auto hd) {
             constexpr int HD = decltype(hd)::value;
@@ -698,19 +870,23 @@ void launch_bulk(const DModel& M, const DLayer* layers, const BulkBuf& B, int p0
         };
         if (M.HD == 64) attn(std::integral_constant<int, 64>());
         else attn(std::integral_constant<int, 128>());
-        gemm<BE_RES>(L.o, B.xq, B.xd, ntt, 1, B.h, nullptr, nullptr, nullptr, 0, s);
+        gemm<BE_RES>(L.o, B.xq, B.xd, ntt, 1, B.h, 0, nullptr, nullptr, s);
         norm(L.fn, nullptr, 0);
-        gemm<BE_GU>(L.gu, B.xq, B.xd, ntt, 1, nullptr, B.aq, B.ad, nullptr, 0, s);
+        // K split while the 64 x 64 tiles are about one per CU (us, split / whole K, at 152 and 280
+        // row groups: 64 tokens 7.4 / 12.0 and 18.1 / 21.1; 128 tokens 13.9 / 13.0 and 28.6 / 24.3;
+        // 512 tokens 32.5 / 26.9 and 73.5 / 56.5)
+        if ((L.gu.rows >> 6) * ntt <= kBulkWgs) gemm<BE_GU>(L.gu, B.xq, B.xd, ntt, 1, nullptr, 0, B.aq, B.ad, s);
+        else gemm_w<BE_GU>(L.gu, B.xq, B.xd, ntt, B.aq, B.ad, nullptr, s);
         ks = ntt * 64 <= kBulkSplitM ? L.d.ks : 0;
-        if (ks) gemm<BE_PART>(L.d, B.aq, B.ad, ntt, ks, B.dpart, nullptr, nullptr, nullptr, kBulkSplitM * E, s);
-        else gemm<BE_RES>(L.d, B.aq, B.ad, ntt, 1, B.h, nullptr, nullptr, nullptr, 0, s);
+        if (ks) gemm<BE_PART>(L.d, B.aq, B.ad, ntt, ks, B.dpart, kBulkSplitM * E, nullptr, nullptr, s);
+        else gemm<BE_RES>(L.d, B.aq, B.ad, ntt, 1, B.h, 0, nullptr, nullptr, s);
     }
     if (!all && !last) return;
     norm(M.out_norm, nullptr, ks);
     // predictions: every token tile, or only the one that holds the last token
     const int tt0 = all ? 0 : ntt - 1, t0 = all ? 0 : m - 1;
-    gemm<BE_LM>(M.lm, B.xq + (size_t)(2 * tt0) * nbE * 1024, B.xd + (size_t)(2 * tt0) * nbE * 32, ntt - tt0, 1, nullptr, nullptr, nullptr,
-                B.cand + (size_t)tt0 * 64 * (M.V / 64), 0, s);
+    gemm_w<BE_LM>(M.lm, B.xq + (size_t)(2 * tt0) * nbE * 1024, B.xd + (size_t)(2 * tt0) * nbE * 32, ntt - tt0, nullptr, nullptr,
+                  B.cand + (size_t)tt0 * 64 * (M.V / 64), s);
     LAUNCH(k_bargmax, m - t0, 64, s, B.cand, M.V / 64, M.V, t0, p0, M.out_tok, M.out_margin);
 }
 

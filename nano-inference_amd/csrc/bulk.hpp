@@ -15,14 +15,14 @@ constexpr int kBulkSplitM = 128;   // up to this many tokens the down GEMM runs 
 // Work buffers of a panel (device memory, kept by the engine). Int8 activations of an
 // nb-block vector per token are stored as the GEMM's MFMA operand: 32-token tiles, per tile
 // and block 64 lanes x 16 codes (lane l: token l % 32, elements 16 (l / 32) .. + 15), with
-// the block scales (fp16 bits) [tile][nb][32] beside them.
+// the block scales (fp16 bits, a word each) [tile][nb][32] beside them.
 struct BulkBuf {
     float* h;                      // [kBulkM][E] residual
     int8_t* xq;                    // [kBulkM/32][E/32][64][16]
-    uint16_t* xd;                  // [kBulkM/32][E/32][32]
+    uint32_t* xd;                  // [kBulkM/32][E/32][32]
     float* qkv;                    // [kBulkM][QKV] projections, then q rotated in place
     int8_t* aq;                    // [kBulkM/32][FF/32][64][16] gate/up output
-    uint16_t* ad;                  // [kBulkM/32][FF/32][32]
+    uint32_t* ad;                  // [kBulkM/32][FF/32][32]
     float* dpart;                  // [ks of down][kBulkSplitM][E]
     float* rec;                    // [kBulkM][NH][max splits][HD + 2] attention split records
     float4* cand;                  // [kBulkM][V/64] argmax candidates
