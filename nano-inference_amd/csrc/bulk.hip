@@ -24,6 +24,7 @@ namespace mi {
 
 #define LAUNCH(kern, grid, block, stream, ...) hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, stream, __VA_ARGS__)
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x32 __attribute__((ext_vector_type(32)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
@@ -51,7 +52,7 @@ BulkSizes bulk_sizes(int E, int FF, int NH, int HD, int QKV, int V, int maxseq, 
     s.aq = M * FF;
     s.ad = M * (FF / 32);
     s.dpart = (size_t)ks_d * kBulkSplitM * E;
-    s.rec = M * NH * nsp * (HD + 2);
+    s.rec = M * NH * nsp * (HD + 4);
     s.cand = M * (V / 64);
     return s;
 }
@@ -563,227 +564,292 @@ __global__ __launch_bounds__(kBThreads) void k_brope(float* qkv, const float* bi
 }
 
 // ------------------------------------------------------------------ attention
-// One workgroup: 32 tokens of one query head against one split (16 chunks of 64 positions).
-// Wave w takes chunks w, w + 4, ...: scores S[position][token] by 32x32x2 f32 MFMAs, one
-// accumulator per chain d mod 4 (k = 0, 1 of an MFMA are d and d + 4 of a chain), the chunk
-// softmax in registers (lane l: token l % 32, half of the chunk's positions; the other half
-// on lane l ^ 32), and, once every chunk's max is known, o[dim][token] by MFMAs over
-// position pairs. The four waves' chunk outputs meet in LDS per round and are merged in
-// chunk order. Rows of D stand for dims NDT*row + dt, so that one lane's V operands of a
-// position are NDT consecutive halves.
-// Record of (token, head, split): o[HD], M, den.
-template <int HD>
-__global__ __launch_bounds__(kBThreads, 1) void k_battn(const float* qkv, int QKV, const __half* kc, const __half* vc,
-                                                        int NH, int G, int m, int p0, int maxseq, int nsp, float scale,
-                                                        float* rec) {
-    constexpr int NJ = HD / 8, NDT = HD / 32;
-    constexpr int kR = kAttnSplit / 4;                       // rounds of four chunks
-    __shared__ float4 ol[4][NDT][4][64];
-    __shared__ float mt[kAttnSplit][32], lt[kAttnSplit][32];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, half = lane >> 5, col = lane & 31;
-    const int ntile = (m + 31) / 32;
-    // the last (longest) tiles first
-    const int h = blockIdx.x % NH, rest = blockIdx.x / NH, sp = rest % nsp, tile = ntile - 1 - rest / nsp;
-    const int tbase = tile * 32, tlast = min(tbase + 31, m - 1);
-    const int nch = (p0 + tlast) / kAttnChunk + 1 - sp * kAttnSplit;    // chunks of this split, if positive
-    if (nch <= 0) return;
-    const int nc = min(nch, kAttnSplit), nr = (nc + 3) / 4;
-    const int tok = min(tbase + col, tlast), pos = p0 + tok, kvh = h / G, prow = p0 + m - 1;
-    const __half* kb = kc + (size_t)kvh * maxseq * HD;
-    const __half* vb = vc + (size_t)kvh * maxseq * HD;
+// mi_expf without its branches (the same value for every input)
+__device__ __forceinline__ float mi_expf_sel(float x) {
+    const float n = __builtin_rintf(__fmul_rn(x, 0x1.715476p+0f));
+    float r = __fmaf_rn(n, -0x1.62e4p-1f, x);
+    r = __fmaf_rn(n, -0x1.7f7d1cp-20f, r);
+    float p = 0x1.a01a02p-13f;
+    p = __fmaf_rn(p, r, 0x1.6c16c2p-10f);
+    p = __fmaf_rn(p, r, 0x1.111112p-7f);
+    p = __fmaf_rn(p, r, 0x1.555556p-5f);
+    p = __fmaf_rn(p, r, 0x1.555556p-3f);
+    p = __fmaf_rn(p, r, 0x1p-1f);
+    p = __fmaf_rn(p, r, 1.0f);
+    p = __fmaf_rn(p, r, 1.0f);
+    p = __builtin_ldexpf(p, (int)n);
+    p = x < -87.0f ? 0.f : p;
+    p = x > 88.72283f ? __builtin_inff() : p;
+    return x != x ? x : p;
+}
 
-    float q[NJ][4];                                          // q[token][8j + 4 half + i]
+// One workgroup, four waves: 16 tokens of one query head against one split (16 chunks of 64
+// positions); two workgroups per CU. An f32 MFMA is a chain of fused multiply-adds in k order,
+// so both canonical contractions run on it:
+//   scores   unit = 32 positions x 16 tokens, units round-robin over the waves: 16x16x4 MFMAs,
+//            one accumulator per chain d mod 4 (k = 0..3 are d, d + 4, d + 8, d + 12 of a chain)
+//   softmax  four lanes per (chunk, token), 16 positions each (position mod 4): the chunk max,
+//            exp and the canonical butterfly sum (in the lane over xor 32, 16, 8, 4, then over
+//            the quad for xor 2, 1)
+//   p.v      wave: HD/4 dims x 16 tokens through all chunks in order by 16x16x4 MFMAs, each
+//            chunk's output merged as it is done (the split's max is known by then), so no
+//            outputs are exchanged
+// Scores and probabilities stay in LDS, 4 KB per chunk: word (position, token) at
+// ((chunk * 4 + position % 4) * 16 + token) * 16 + position / 4, the four-word groups swizzled
+// (ps_at).
+// K and V rows are read without a clamp: rows past the panel are masked (scores) or meet
+// p = 0 (see below), and the cache is allocated a chunk longer than its last row.
+// nsp == 1: o / den goes straight into the O GEMM's int8 operand; otherwise the record of
+// (token, head, split): o[HD], M, den.
+// Bound by the MFMAs and the vector unit, which f32 MFMAs hold up. Per layer of the 1.5B shape
+// with 512-token panels: 64 tokens 8.5 us, 512 tokens 30, tokens 1024..1535 71, 2048..2559
+// 112; 32-token workgroups (one per CU) 9.9, 34, 116, 132; the waves on whole chunks, their
+// outputs exchanged, everything unrolled (an 8k-line loop body) 23, 41, 105, 178.
+constexpr int kAT = 16, kAWaves = 4, kAThreads = 64 * kAWaves;
+__device__ __forceinline__ int ps_at(int c, int pos, int tok) {
+    const int k = pos & 3, i = pos >> 2;
+    return ((c * 4 + k) * kAT + tok) * 16 + ((((i >> 2) ^ (tok >> 2) ^ k) & 3) << 2) + (i & 3);
+}
+template <int HD>
+__global__ __launch_bounds__(kAThreads, 2) void k_battn(const float* qkv, int QKV, const __half* kc, const __half* vc,
+                                                        int NH, int G, int m, int p0, int maxseq, int nsp, float scale,
+                                                        float* rec, int nb, int8_t* xq, uint32_t* xd) {
+    constexpr int NJ = HD / 16, NU = HD / 64;
+    __shared__ __align__(16) float ps[kAttnSplit * 4 * kAT * 16];
+    __shared__ float mt[kAttnSplit][kAT], lt[kAttnSplit][kAT], wt[kAttnSplit][kAT], amx[4][kAT];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int ntile = (m + kAT - 1) / kAT;
+    // whole splits before the ragged last one, late (long) tiles first
+    const int h = blockIdx.x % NH, rest = blockIdx.x / NH, sp = rest / ntile, tile = ntile - 1 - (rest - sp * ntile);
+    const int tbase = tile * kAT, tlast = min(tbase + kAT - 1, m - 1), c0 = sp * kAttnSplit;
+    const int nch = (p0 + tlast) / kAttnChunk + 1 - c0;      // chunks of this split, if positive
+    if (nch <= 0) return;
+    const int nc = min(nch, kAttnSplit), kvh = h / G;
+    const __half* kb = kc + ((size_t)kvh * maxseq + c0 * kAttnChunk) * HD;
+    const __half* vb = vc + ((size_t)kvh * maxseq + c0 * kAttnChunk) * HD;
+    const int kk = lane >> 4, tk = lane & 15, tok = min(tbase + tk, tlast), pos = p0 + tok;
+    const int nct = min(pos / kAttnChunk + 1 - c0, kAttnSplit);   // this token's chunks of the split, may be <= 0
+
+    // p.v: wave's dims d0 .., dim d0 + NU r + u on row r of D tile u; a lane's V rows are 4i + kk
+    const int d0 = wave * 16 * NU;
+    typedef typename std::conditional<NU == 2, uint32_t, uint16_t>::type VT;
+    typedef uint32_t VR;                                     // in a whole register
+    const int voff = kk * HD + NU * tk;
+    auto vld = [&](int c, int i) {
+        return (VR)*reinterpret_cast<const VT*>(vb + ((size_t)c * kAttnChunk + 4 * i) * HD + d0 + voff);
+    };
+    auto vf = [](VR w, int u) { return u ? h2f_hi(w) : h2f_lo(w); };
+    VR vr[16];
 #pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        const float4 v = *reinterpret_cast<const float4*>(qkv + (size_t)tok * QKV + h * HD + 8 * j + 4 * half);
-        q[j][0] = v.x; q[j][1] = v.y; q[j][2] = v.z; q[j][3] = v.w;
-    }
-    float p[kR][2][16];                                      // scores, then probabilities, of the wave's chunks
+    for (int i = 0; i < 16; i++) vr[i] = vld(0, i);          // the first chunk's, while the scores run
+    asm volatile("" ::: "memory");
+
+    {   // scores
+        float q[NJ][4];                                      // q[token][16j + 4 kk + i]
 #pragma unroll
-    for (int r = 0; r < kR; r++) {
-        const int ci = 4 * r + wave;
-        if (ci < nc) {
-            const int t0 = (sp * kAttnSplit + ci) * kAttnChunk;
-            f32x16 s[2][4];
+        for (int j = 0; j < NJ; j++) {
+            const float4 v = *reinterpret_cast<const float4*>(qkv + (size_t)tok * QKV + h * HD + 16 * j + 4 * kk);
+            q[j][0] = v.x; q[j][1] = v.y; q[j][2] = v.z; q[j][3] = v.w;
+        }
+        // a unit's K rows, all at once (a line's pieces find it in the L1), a unit ahead
+        uint2 kr[2][NJ], kn[2][NJ];
+        const int koff = tk * HD + 4 * kk;
+        auto kload = [&](uint2 (&k)[2][NJ], int unit) {
 #pragma unroll
-            for (int u = 0; u < 2; u++)
+            for (int t = 0; t < 2; t++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) s[u][i] = f32x16{};
-            const __half* k0 = kb + (size_t)min(t0 + col, prow) * HD + 4 * half;
-            const __half* k1 = kb + (size_t)min(t0 + 32 + col, prow) * HD + 4 * half;
+                for (int j = 0; j < NJ; j++)
+                    k[t][j] = *reinterpret_cast<const uint2*>(kb + (size_t)(unit * 32 + 16 * t) * HD + 16 * j + koff);
+            asm volatile("" ::: "memory");
+        };
+        if (wave < 2 * nc) kload(kr, wave);
+        for (int unit = wave; unit < 2 * nc; unit += kAWaves) {
+            kload(kn, min(unit + kAWaves, 2 * nc - 1));
+            f32x4 s[2][4];
 #pragma unroll
-            for (int j = 0; j < NJ; j++) {
-                const uint2 a = *reinterpret_cast<const uint2*>(k0 + 8 * j);
-                const uint2 b = *reinterpret_cast<const uint2*>(k1 + 8 * j);
-                const float av[4] = {h2f_lo(a.x), h2f_hi(a.x), h2f_lo(a.y), h2f_hi(a.y)};
-                const float bv[4] = {h2f_lo(b.x), h2f_hi(b.x), h2f_lo(b.y), h2f_hi(b.y)};
+            for (int t = 0; t < 2; t++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    s[0][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], q[j][i], s[0][i], 0, 0, 0);
-                    s[1][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[i], q[j][i], s[1][i], 0, 0, 0);
+                for (int i = 0; i < 4; i++) s[t][i] = f32x4{};
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    uint2 w = kr[t][j];
+                    asm volatile("" : "+v"(w.x), "+v"(w.y));     // its wait stays here
+                    const float kv[4] = {h2f_lo(w.x), h2f_hi(w.x), h2f_lo(w.y), h2f_hi(w.y)};
+#pragma unroll
+                    for (int i = 0; i < 4; i++) s[t][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i], q[j][i], s[t][i], 0, 0, 0);
                 }
-            }
-            float mx = -__builtin_inff();
-            bool any = false;
 #pragma unroll
-            for (int u = 0; u < 2; u++)
+            for (int t = 0; t < 2; t++)
 #pragma unroll
-                for (int j = 0; j < 16; j++) {
-                    const bool ok = t0 + 32 * u + drow(j, half) <= pos;
-                    const float v = __fmul_rn(__fadd_rn(__fadd_rn(s[u][0][j], s[u][1][j]), __fadd_rn(s[u][2][j], s[u][3][j])), scale);
-                    p[r][u][j] = ok ? v : -__builtin_inff();
-                    mx = any ? fmaxf(mx, p[r][u][j]) : p[r][u][j];
-                    any = true;
+                for (int j = 0; j < NJ; j++) kr[t][j] = kn[t][j];
+            // the lane holds positions 16t + 4 kk + r of the unit, token tk
+            const int c = unit >> 1, o = 32 * (unit & 1) + 4 * kk, t0 = (c0 + c) * kAttnChunk;
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float v = __fmul_rn(__fadd_rn(__fadd_rn(s[t][0][r], s[t][1][r]), __fadd_rn(s[t][2][r], s[t][3][r])), scale);
+                    ps[ps_at(c, o + 16 * t + r, tk)] = t0 + o + 16 * t + r <= pos ? v : -__builtin_inff();
                 }
-            float x, y;
-            pair32(mx, x, y);
-            mx = fmaxf(x, y);
-            float e1[2][16];
-#pragma unroll
-            for (int u = 0; u < 2; u++)
-#pragma unroll
-                for (int j = 0; j < 16; j++) {
-                    const bool ok = t0 + 32 * u + drow(j, half) <= pos;
-                    p[r][u][j] = ok ? mi_expf(__fsub_rn(p[r][u][j], mx)) : 0.f;
-                    e1[u][j] = p[r][u][j];
-                }
-            // the canonical butterfly over positions: xor 32 (u), 16 and 8 (j / 4), 4 (lane
-            // half), 2 and 1 (j % 4)
-            float b4[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                float z[4];
-#pragma unroll
-                for (int j = 0; j < 4; j++) z[j] = __fadd_rn(e1[0][4 * j + i], e1[1][4 * j + i]);
-                const float y0 = __fadd_rn(z[0], z[2]), y1 = __fadd_rn(z[1], z[3]);
-                pair32(__fadd_rn(y0, y1), x, y);
-                b4[i] = __fadd_rn(x, y);
-            }
-            const float ls = __fadd_rn(__fadd_rn(b4[0], b4[2]), __fadd_rn(b4[1], b4[3]));
-            if (half == 0) {
-                mt[ci][col] = mx;
-                lt[ci][col] = ls;
-            }
         }
     }
     __syncthreads();
-    // this token's chunks of the split, their max, and the merge in chunk order
-    const int nct = min(pos / kAttnChunk + 1 - sp * kAttnSplit, kAttnSplit);     // may be <= 0 for the tile's first tokens
-    float Ms = mt[0][col];
+    for (int it = tid; it < nc * 4 * kAT; it += kAThreads) { // softmax
+        const int k = it & 3, t2 = (it >> 2) & (kAT - 1), c = it / (4 * kAT);
+        const int last = p0 + min(tbase + t2, tlast) - (c0 + c) * kAttnChunk;     // the token's own offset in the chunk
+        float v[16];
 #pragma unroll
-    for (int c = 1; c < kAttnSplit; c++)
-        if (c < nct) Ms = fmaxf(Ms, mt[c][col]);
-    float den = 0.f, as[4 * NDT];
+        for (int i = 0; i < 4; i++) {
+            const float4 f = *reinterpret_cast<const float4*>(ps + ps_at(c, 16 * i + k, t2));
+            v[4 * i] = f.x; v[4 * i + 1] = f.y; v[4 * i + 2] = f.z; v[4 * i + 3] = f.w;
+        }
+        float mx = v[0];
 #pragma unroll
-    for (int j = 0; j < 4 * NDT; j++) as[j] = 0.f;
+        for (int i = 1; i < 16; i++) mx = fmaxf(mx, v[i]);
+        mx = fmaxf(mx, dppf<kDppXor2>(mx));
+        mx = fmaxf(mx, dppf<kDppXor1>(mx));
 #pragma unroll
-    for (int r = 0; r < kR; r++) {
-        if (r < nr) {
-            const int ci = 4 * r + wave;
-            if (ci < nc) {
-                const int t0 = (sp * kAttnSplit + ci) * kAttnChunk;
-                f32x16 o[NDT];
+        for (int i = 0; i < 16; i++) {
+            float e = mi_expf_sel(__fsub_rn(v[i], mx));
+            asm("" : "+v"(e));                               // a select, not a branch around the exp
+            v[i] = 4 * i + k <= last ? e : 0.f;
+        }
 #pragma unroll
-                for (int d = 0; d < NDT; d++) o[d] = f32x16{};
+        for (int i = 0; i < 4; i++)
+            *reinterpret_cast<float4*>(ps + ps_at(c, 16 * i + k, t2)) = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
 #pragma unroll
-                for (int u = 0; u < 2; u++)
+        for (int d = 8; d >= 1; d >>= 1)                     // xor 32, 16, 8, 4 over positions
 #pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        // positions 32u + 8j .. + 7: half 0 holds 0..3, half 1 4..7; the MFMA
-                        // wants pairs (0,1), (2,3), (4,5), (6,7) across the halves
-                        const auto sa = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[r][u][4 * j]), __float_as_uint(p[r][u][4 * j + 1]), false, false);
-                        const auto sb = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[r][u][4 * j + 2]), __float_as_uint(p[r][u][4 * j + 3]), false, false);
-                        const float pb[4] = {__uint_as_float(sa[0]), __uint_as_float(sb[0]), __uint_as_float(sa[1]), __uint_as_float(sb[1])};
-#pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            const int row = min(t0 + 32 * u + 8 * j + 2 * i + half, prow);
-                            const __half* v = vb + (size_t)row * HD + NDT * col;
-                            float vv[NDT];
-                            if constexpr (NDT == 4) {
-                                const uint2 w = *reinterpret_cast<const uint2*>(v);
-                                vv[0] = h2f_lo(w.x); vv[1] = h2f_hi(w.x); vv[2] = h2f_lo(w.y); vv[3] = h2f_hi(w.y);
-                            } else {
-                                const uint32_t w = *reinterpret_cast<const uint32_t*>(v);
-                                vv[0] = h2f_lo(w); vv[1] = h2f_hi(w);
-                            }
-#pragma unroll
-                            for (int d = 0; d < NDT; d++) o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[d], pb[i], o[d], 0, 0, 0);
-                        }
-                    }
-                // A position past a token's own has p = 0, which adds exactly nothing unless its V
-                // holds an infinity or NaN (0 * inf): the canonical chain stops before it. So where
-                // the chunk reaches past the tile's first token and a result is NaN, the chain runs
-                // again one position at a time, each result kept only for the tokens that see it.
-                if (t0 + kAttnChunk - 1 > p0 + tbase) {
-                    bool nan = false;
-#pragma unroll
-                    for (int d = 0; d < NDT; d++)
-#pragma unroll
-                        for (int j = 0; j < 16; j++) nan |= o[d][j] != o[d][j];
-                    if (__builtin_amdgcn_ballot_w64(nan)) {
-                        float* ps = reinterpret_cast<float*>(&ol[wave][0][0][0]);       // [64 positions][32 tokens]
-#pragma unroll
-                        for (int u = 0; u < 2; u++)
-#pragma unroll
-                            for (int j = 0; j < 16; j++) ps[(32 * u + drow(j, half)) * 32 + col] = p[r][u][j];
-                        __builtin_amdgcn_s_waitcnt(0xC07F);
-#pragma unroll
-                        for (int d = 0; d < NDT; d++) o[d] = f32x16{};
-#pragma unroll 1
-                        for (int k = 0; k < kAttnChunk; k++) {
-                            const bool on = (k & 1) == half, sees = t0 + k <= pos;
-                            const float pk = on ? ps[k * 32 + col] : 0.f;
-                            const __half* v = vb + (size_t)min(t0 + k, prow) * HD + NDT * col;
-#pragma unroll
-                            for (int d = 0; d < NDT; d++) {
-                                const f32x16 z = __builtin_amdgcn_mfma_f32_32x32x2f32(on ? __half2float(v[d]) : 0.f, pk, o[d], 0, 0, 0);
-#pragma unroll
-                                for (int j = 0; j < 16; j++) o[d][j] = sees ? z[j] : o[d][j];
-                            }
-                        }
-                        __builtin_amdgcn_s_waitcnt(0xC07F);
-                    }
-                }
-#pragma unroll
-                for (int d = 0; d < NDT; d++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++)
-                        ol[wave][d][j][lane] = make_float4(o[d][4 * j], o[d][4 * j + 1], o[d][4 * j + 2], o[d][4 * j + 3]);
-            }
-            __syncthreads();
-            // wave w merges quarter w of the 4 NDT float4 a lane holds
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int c = 4 * r + i;
-                if (c < nct) {
-                    const float wc = mi_expf(__fsub_rn(mt[c][col], Ms));
-                    den = __fmaf_rn(lt[c][col], wc, den);
-#pragma unroll
-                    for (int k = 0; k < NDT; k++) {
-                        const int f = wave * NDT + k;
-                        const float4 v = ol[i][f >> 2][f & 3][lane];
-                        as[4 * k] = __fmaf_rn(v.x, wc, as[4 * k]);
-                        as[4 * k + 1] = __fmaf_rn(v.y, wc, as[4 * k + 1]);
-                        as[4 * k + 2] = __fmaf_rn(v.z, wc, as[4 * k + 2]);
-                        as[4 * k + 3] = __fmaf_rn(v.w, wc, as[4 * k + 3]);
-                    }
-                }
-            }
-            __syncthreads();
+            for (int i = 0; i < d; i++) v[i] = __fadd_rn(v[i], v[i + d]);
+        float l = __fadd_rn(v[0], dppf<kDppXor2>(v[0]));
+        l = __fadd_rn(l, dppf<kDppXor1>(l));
+        if (k == 0) {
+            mt[c][t2] = mx;
+            lt[c][t2] = l;
         }
     }
-    if (tbase + col > tlast || nct <= 0) return;
-    float* rp = rec + (((size_t)tok * NH + h) * nsp + sp) * (HD + 2);
-#pragma unroll
-    for (int k = 0; k < NDT; k++) {
-        const int f = wave * NDT + k, d = f >> 2, j = f & 3;
-#pragma unroll
-        for (int i = 0; i < 4; i++) rp[NDT * (8 * j + 4 * half + i) + d] = as[4 * k + i];
+    __syncthreads();
+    {   // chunk weights exp(m_c - M) of the split: a thread per (chunk, token)
+        const int c = tid / kAT, t2 = tid & (kAT - 1);
+        const int n2 = min((p0 + min(tbase + t2, tlast)) / kAttnChunk + 1 - c0, kAttnSplit);
+        float M = mt[0][t2];
+        for (int i = 1; i < n2; i++) M = fmaxf(M, mt[i][t2]);
+        if (c < n2) wt[c][t2] = mi_expf_sel(__fsub_rn(mt[c][t2], M));
+        if (c == 0) amx[0][t2] = M;
     }
-    if (wave == 0 && half == 0) {
-        rp[HD] = Ms;
-        rp[HD + 1] = den;
+    __syncthreads();
+    const float Ms = amx[0][tk];
+
+    float den = 0.f;
+    f32x4 as[NU];
+#pragma unroll
+    for (int u = 0; u < NU; u++) as[u] = f32x4{};
+    for (int c = 0; c < nc; c++) {
+        f32x4 o[NU];
+#pragma unroll
+        for (int u = 0; u < NU; u++) o[u] = f32x4{};
+        const int cn = min(c + 1, nc - 1);
+        float4 pv[4];
+#pragma unroll
+        for (int i4 = 0; i4 < 4; i4++) pv[i4] = *reinterpret_cast<const float4*>(ps + ps_at(c, 16 * i4 + kk, tk));
+#pragma unroll
+        for (int i4 = 0; i4 < 4; i4++) {
+            const float pb[4] = {pv[i4].x, pv[i4].y, pv[i4].z, pv[i4].w};
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                VR w = vr[4 * i4 + i];
+                asm volatile("" : "+v"(w));
+                vr[4 * i4 + i] = vld(cn, 4 * i4 + i);        // the next chunk's, a chunk ahead
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int u = 0; u < NU; u++) o[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf(w, u), pb[i], o[u], 0, 0, 0);
+            }
+        }
+        // A position past a token's own has p = 0, which adds exactly nothing unless its V
+        // holds an infinity or NaN (0 * inf): the canonical chain stops before it. So where
+        // the chunk reaches past the tile's first token and a result is NaN, the chain runs
+        // again one position at a time, each result kept only for the tokens that see it.
+        if ((c0 + c + 1) * kAttnChunk - 1 > p0 + tbase) {
+            bool nan = false;
+#pragma unroll
+            for (int u = 0; u < NU; u++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) nan |= o[u][j] != o[u][j];
+            if (__builtin_amdgcn_ballot_w64(nan)) {
+#pragma unroll
+                for (int u = 0; u < NU; u++) o[u] = f32x4{};
+#pragma unroll 1
+                for (int k = 0; k < kAttnChunk; k++) {
+                    const bool on = (k & 3) == kk, sees = (c0 + c) * kAttnChunk + k <= pos;
+                    const float pk = on ? ps[ps_at(c, k, tk)] : 0.f;
+                    const VR w = vld(c, k >> 2);
+#pragma unroll
+                    for (int u = 0; u < NU; u++) {
+                        const f32x4 z = __builtin_amdgcn_mfma_f32_16x16x4f32(on ? vf(w, u) : 0.f, pk, o[u], 0, 0, 0);
+#pragma unroll
+                        for (int j = 0; j < 4; j++) o[u][j] = sees ? z[j] : o[u][j];
+                    }
+                }
+            }
+        }
+        if (c < nct) {
+            const float w = wt[c][tk];
+            den = __fmaf_rn(lt[c][tk], w, den);
+#pragma unroll
+            for (int u = 0; u < NU; u++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) as[u][j] = __fmaf_rn(o[u][j], w, as[u][j]);
+        }
     }
+    // the lane's 4 NU consecutive dims, from d0 + 4 NU kk
+    float out[4 * NU];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int u = 0; u < NU; u++) out[NU * j + u] = as[u][j];
+    const bool mine = tbase + tk <= tlast && nct > 0;
+    if (nsp > 1) {
+        if (!mine) return;
+        float* rp = rec + (((size_t)tok * NH + h) * nsp + sp) * (HD + 4);
+#pragma unroll
+        for (int u = 0; u < NU; u++)
+            *reinterpret_cast<float4*>(rp + d0 + 4 * NU * kk + 4 * u) = make_float4(out[4 * u], out[4 * u + 1], out[4 * u + 2], out[4 * u + 3]);
+        if (wave == 0 && kk == 0) {
+            rp[HD] = Ms;
+            rp[HD + 1] = den;
+        }
+        return;
+    }
+    float mx = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4 * NU; e++) {
+        out[e] = __fdiv_rn(out[e], den);
+        mx = fmaxf(mx, fabsf(out[e]));
+    }
+    float x, y;
+    pair32(mx, x, y);
+    mx = fmaxf(x, y);
+    pair16(mx, x, y);
+    mx = fmaxf(x, y);
+    if constexpr (NU == 1) {                                 // a block's 32 dims lie on two waves
+        __syncthreads();
+        amx[wave][tk] = mx;
+        __syncthreads();
+        mx = fmaxf(mx, amx[wave ^ 1][tk]);
+    }
+    if (!mine) return;
+    const float inv = mx > 0.f ? __fdiv_rn(127.f, mx) : 0.f;
+    const int e0 = h * HD + d0 + 4 * NU * kk;
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+        uint32_t w = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) w |= (uint32_t)(__float2int_rn(__fmul_rn(out[4 * u + i], inv)) & 0xFF) << (8 * i);
+        *reinterpret_cast<uint32_t*>(xq + bx_at(nb, tok, e0 >> 5, (e0 & 31) + 4 * u)) = w;
+    }
+    if ((e0 & 31) == 0) xd[bd_at(nb, tok, e0 >> 5)] = f2h_bits(__fdiv_rn(mx, 127.f));
 }
 
 // split merge of (token, head) by one wave (lane = dims 64e + lane), then int8 blocks into
@@ -796,7 +862,7 @@ __global__ __launch_bounds__(kBThreads) void k_bcomb(const float* rec, int NH, i
     if (item >= m * NH) return;
     const int t = item / NH, h = item - t * NH;
     const int ns = (p0 + t) / (kAttnChunk * kAttnSplit) + 1;
-    const float* r = rec + (size_t)item * nsp * (HD + 2);
+    const float* r = rec + (size_t)item * nsp * (HD + 4);
     float den, o[DPL];
     if (ns == 1) {
         den = r[HD + 1];
@@ -804,13 +870,13 @@ __global__ __launch_bounds__(kBThreads) void k_bcomb(const float* rec, int NH, i
         for (int e = 0; e < DPL; e++) o[e] = r[64 * e + lane];
     } else {
         float Mx = -__builtin_inff();
-        for (int s = lane; s < ns; s += 64) Mx = fmaxf(Mx, r[(size_t)s * (HD + 2) + HD]);
+        for (int s = lane; s < ns; s += 64) Mx = fmaxf(Mx, r[(size_t)s * (HD + 4) + HD]);
         Mx = wave_max(Mx);
         den = 0.f;
 #pragma unroll
         for (int e = 0; e < DPL; e++) o[e] = 0.f;
         for (int s = 0; s < ns; s++) {
-            const float* q = r + (size_t)s * (HD + 2);
+            const float* q = r + (size_t)s * (HD + 4);
             const float w = mi_expf(__fsub_rn(q[HD], Mx));
             den = __fmaf_rn(q[HD + 1], w, den);
 #pragma unroll
@@ -864,9 +930,10 @@ void launch_bulk(const DModel& M, const DLayer* layers, const BulkBuf& B, int p0
             const size_t threads = (size_t)m * (M.NH + 2 * M.NKV) * (HD / 2);
             LAUNCH((k_brope<HD>), (unsigned)((threads + kBThreads - 1) / kBThreads), kBThreads, s, B.qkv, L.bqkv, M.rope, M.NH,
                    M.NKV, M.QKV, m, p0, M.maxseq, M.kc + kv, M.vc + kv);
-            LAUNCH((k_battn<HD>), (unsigned)(M.NH * nsp * ((m + 31) / 32)), kBThreads, s, B.qkv, M.QKV, M.kc + kv, M.vc + kv,
-                   M.NH, M.G, m, p0, M.maxseq, nsp, M.scale, B.rec);
-            LAUNCH((k_bcomb<HD>), (m * M.NH + 3) / 4, kBThreads, s, B.rec, M.NH, m, p0, nsp, nbE, B.xq, B.xd);
+            LAUNCH((k_battn<HD>), (unsigned)(M.NH * nsp * ((m + kAT - 1) / kAT)), kAThreads, s, B.qkv, M.QKV, M.kc + kv, M.vc + kv,
+                   M.NH, M.G, m, p0, M.maxseq, nsp, M.scale, B.rec, nbE, B.xq, B.xd);
+            if (nsp > 1)
+                LAUNCH((k_bcomb<HD>), (m * M.NH + 3) / 4, kBThreads, s, B.rec, M.NH, m, p0, nsp, nbE, B.xq, B.xd);
         };
         if (M.HD == 64) attn(std::integral_constant<int, 64>());
         else attn(std::integral_constant<int, 128>());

@@ -24,7 +24,7 @@ struct BulkBuf {
     int8_t* aq;                    // [kBulkM/32][FF/32][64][16] gate/up output
     uint32_t* ad;                  // [kBulkM/32][FF/32][32]
     float* dpart;                  // [ks of down][kBulkSplitM][E]
-    float* rec;                    // [kBulkM][NH][max splits][HD + 2] attention split records
+    float* rec;                    // [kBulkM][NH][max splits][HD + 4] attention split records
     float4* cand;                  // [kBulkM][V/64] argmax candidates
 };
 struct BulkSizes { size_t h, xq, xd, qkv, aq, ad, dpart, rec, cand; };   // in elements

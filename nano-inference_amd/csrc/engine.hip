@@ -495,7 +495,9 @@ static int load_impl(mi_engine* e, const char* path) {
     M.arec = attn_record_floats(e->HD);
     const size_t NL = (size_t)e->NL;
     const Dims D = step_dims(e->NL, e->E, e->FF, e->NH, e->NKV, e->V, e->maxseq, e->cb, e->ks, e->n_cu);
-    if ((rc = alloc_buf(e, &M.kc, lay::kv_size(D))) || (rc = alloc_buf(e, &M.vc, lay::kv_size(D))) ||
+    // the prompt panels read whole attention chunks: up to a chunk past the last row
+    const size_t kv_pad = (size_t)kAttnChunk * e->HD;
+    if ((rc = alloc_buf(e, &M.kc, lay::kv_size(D) + kv_pad)) || (rc = alloc_buf(e, &M.vc, lay::kv_size(D) + kv_pad)) ||
         (rc = alloc_buf(e, &M.tokbuf, (size_t)e->maxseq + 1)) ||
         (rc = alloc_buf(e, &M.hbuf, lay::hbuf_size(D))) ||
         (rc = alloc_buf(e, &M.qkv_part, lay::qkv_part_size(D))) ||
