@@ -40,8 +40,8 @@ typedef struct mi_engine mi_engine;
 typedef struct mi_opts {
     int32_t max_ctx;       /* KV cache capacity in positions (0: 4096) */
     int32_t tchunk;        /* prompt tokens per step, 1..8. At 8 (the default) prompts of 17 tokens and more
-                              take panels of up to 512 tokens per pass over the weights instead (same
-                              bits; 512 tokens of the 1.5B shape: 84.1 -> 6.6 ms) */
+                              take panels of up to 2048 tokens per pass over the weights instead (same
+                              bits; 512 tokens of the 1.5B shape: 84.1 -> 4.5 ms) */
     int32_t spec;          /* n-gram speculative decoding inside mi_generate: 0 off; 1 the host drafts,
                               launches each verify step and commits its result; 2 the whole loop runs
                               on the device (mega.cu:863-895: each persistent verify launch commits

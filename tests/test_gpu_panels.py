@@ -1,10 +1,10 @@
 """GPU parity of the prompt panels (csrc/bulk.hip): mi_prefill and mi_teacher run prompts of
-17 tokens and more in panels of up to 512 tokens. Bar: the same bits as one multi-token step
+17 tokens and more in panels of up to 2048 tokens. Bar: the same bits as one multi-token step
 per 7 tokens (tchunk=7, itself bit-identical to single steps and the q8act oracle), in the
 predictions, the margins and, through a step's logits, the K/V the panel left.
 
 Lengths sit on the edges of the 32-token tiles, the 64-token GEMM tiles, the panel whose down
-matrix is split over workgroups (128), the panel (512) and the attention split (1024)."""
+matrix is split over workgroups (128), the attention split (1024) and the panel (2048)."""
 import sys
 
 import numpy as np
@@ -36,13 +36,13 @@ def pair(request):
     """an engine that runs panels and one that runs 7-token steps, the same model"""
     shape = SHAPES[request.param]
     path = synth_cached("panel-" + request.param, shape, 31, qk_bias_std=2.0, norm_offset=1.0)
-    a, b = minfer.Engine(path, max_ctx=1152), minfer.Engine(path, max_ctx=1152, tchunk=7)
+    a, b = minfer.Engine(path, max_ctx=2112), minfer.Engine(path, max_ctx=2112, tchunk=7)
     yield shape, a, b
     a.close()
     b.close()
 
 
-@pytest.mark.parametrize("n", [17, 32, 33, 63, 64, 65, 128, 129, 257, 512, 513, 1024, 1025, 1151])
+@pytest.mark.parametrize("n", [17, 32, 33, 63, 64, 65, 128, 129, 257, 512, 513, 1024, 1025, 1151, 2048, 2049])
 def test_panel_bit_identical(pair, n):
     shape, a, b = pair
     print("[gpu-panel] n", n, flush=True)
