@@ -39,7 +39,7 @@ typedef struct mi_engine mi_engine;
  * SPEC_SLOPE (:1022) -> spec_slope; maxseq = P + n_gen + TMAX (:1023) -> max_ctx. */
 typedef struct mi_opts {
     int32_t max_ctx;       /* KV cache capacity in positions (0: 4096) */
-    int32_t tchunk;        /* prompt tokens per step, 1..8. At 8 (the default) prompts of 17 tokens and more
+    int32_t tchunk;        /* prompt tokens per step, 1..8. At 8 (the default) prompts of 9 tokens and more
                               take panels of up to 2048 tokens per pass over the weights instead (same
                               bits; 512 tokens of the 1.5B shape: 84.1 -> 4.5 ms) */
     int32_t spec;          /* n-gram speculative decoding inside mi_generate: 0 off; 1 the host drafts,

@@ -472,58 +472,70 @@ __global__ __launch_bounds__(64) void k_bargmax(const float4* cand, int ng, int 
 }
 
 // ------------------------------------------------------------------ residual, norm, quant
-// One wave per token: h (layer 0: the embedding row) + the down partials in order, written
-// back; RMSNorm and int8 quantisation into the GEMM operand. Lane l holds elements
-// 256j + 4l .. + 3, the order of the canonical sum of squares (rms_scale).
+// One workgroup per token: h (layer 0: the embedding row) + the down partials in order,
+// written back; RMSNorm and int8 quantisation into the GEMM operand. Thread i holds elements
+// 4i .. + 3 (and those 1024 further on); the row meets in LDS, where every wave takes the
+// canonical sum of squares (lane l: elements 256j + 4l + i over j, then i). A wave per token
+// was a chain of its partials' loads on 16 CUs at 64 tokens: 20.4 us with the 10 partials of
+// the 1.5B shape.
 __global__ __launch_bounds__(kBThreads) void k_bnorm(int n, float eps, const float* w, float* h, const float* emb,
-                                                     const int32_t* tok, const float* part, int ks, int m, int8_t* xq,
+                                                     const int32_t* tok, const float* part, int ks, int8_t* xq,
                                                      uint32_t* xd) {
-    constexpr int NJ = kBMaxE / 256;
-    const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (t >= m) return;
+    constexpr int NI = kBMaxE / (4 * kBThreads);
+    __shared__ __align__(16) float row[kBMaxE];
+    const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     const float* src = emb ? emb + (size_t)tok[t] * n : h + (size_t)t * n;
-    float4 x[NJ];
-    float a = 0.f;
+    float4 x[NI], wv[NI];
 #pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        const int e = 256 * j + 4 * lane;
-        x[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int i = 0; i < NI; i++) {
+        const int e = 4 * (tid + i * kBThreads);
+        x[i] = wv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (e < n) {
-            x[j] = *reinterpret_cast<const float4*>(src + e);
+            x[i] = *reinterpret_cast<const float4*>(src + e);
+            wv[i] = *reinterpret_cast<const float4*>(w + e);
             if (ks > 0) {
-                float4 s = *reinterpret_cast<const float4*>(part + (size_t)t * n + e);
-                for (int k = 1; k < ks; k++) {
-                    const float4 p = *reinterpret_cast<const float4*>(part + ((size_t)k * kBulkSplitM + t) * n + e);
+                const float* pt = part + (size_t)t * n + e;
+                const size_t step = (size_t)kBulkSplitM * n;
+                float4 s = *reinterpret_cast<const float4*>(pt);
+                auto add = [&](float4 p) {
                     s = make_float4(__fadd_rn(s.x, p.x), __fadd_rn(s.y, p.y), __fadd_rn(s.z, p.z), __fadd_rn(s.w, p.w));
+                };
+                int k = 1;
+                for (; k + 3 <= ks; k += 3) {                // three loads ahead of their adds
+                    const float4 a = *reinterpret_cast<const float4*>(pt + k * step);
+                    const float4 b = *reinterpret_cast<const float4*>(pt + (k + 1) * step);
+                    const float4 c = *reinterpret_cast<const float4*>(pt + (k + 2) * step);
+                    add(a);
+                    add(b);
+                    add(c);
                 }
-                x[j] = make_float4(__fadd_rn(x[j].x, s.x), __fadd_rn(x[j].y, s.y), __fadd_rn(x[j].z, s.z),
-                                   __fadd_rn(x[j].w, s.w));
+                for (; k < ks; k++) add(*reinterpret_cast<const float4*>(pt + k * step));
+                x[i] = make_float4(__fadd_rn(x[i].x, s.x), __fadd_rn(x[i].y, s.y), __fadd_rn(x[i].z, s.z), __fadd_rn(x[i].w, s.w));
             }
-            if (emb || ks > 0) *reinterpret_cast<float4*>(h + (size_t)t * n + e) = x[j];
+            if (emb || ks > 0) *reinterpret_cast<float4*>(h + (size_t)t * n + e) = x[i];
         }
+        *reinterpret_cast<float4*>(row + e) = x[i];          // zeros past n: fma(0, 0, a) = a
     }
-#pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        a = __fmaf_rn(x[j].x, x[j].x, a); a = __fmaf_rn(x[j].y, x[j].y, a);
-        a = __fmaf_rn(x[j].z, x[j].z, a); a = __fmaf_rn(x[j].w, x[j].w, a);
+    __syncthreads();
+    float a = 0.f;
+    for (int j = 0; 256 * j < n; j++) {
+        const float4 u = *reinterpret_cast<const float4*>(row + 256 * j + 4 * lane);
+        a = __fmaf_rn(u.x, u.x, a); a = __fmaf_rn(u.y, u.y, a);
+        a = __fmaf_rn(u.z, u.z, a); a = __fmaf_rn(u.w, u.w, a);
     }
     a = bfly_sum64(a);
     const float sc = __fdiv_rn(1.0f, __builtin_sqrtf(__fadd_rn(__fdiv_rn(a, (float)n), eps)));
     const int nb = n / 32;
 #pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        if (256 * j >= n) break;
-        const int e = 256 * j + 4 * lane;
-        const bool own = e < n;
-        const float4 wv = own ? *reinterpret_cast<const float4*>(w + e) : make_float4(0.f, 0.f, 0.f, 0.f);
-        float4 y = make_float4(__fmul_rn(__fmul_rn(x[j].x, sc), wv.x), __fmul_rn(__fmul_rn(x[j].y, sc), wv.y),
-                               __fmul_rn(__fmul_rn(x[j].z, sc), wv.z), __fmul_rn(__fmul_rn(x[j].w, sc), wv.w));
-        if (!own) y = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int i = 0; i < NI; i++) {
+        const int e = 4 * (tid + i * kBThreads);             // a block is 8 lanes: all in or all past n
+        float4 y = make_float4(__fmul_rn(__fmul_rn(x[i].x, sc), wv[i].x), __fmul_rn(__fmul_rn(x[i].y, sc), wv[i].y),
+                               __fmul_rn(__fmul_rn(x[i].z, sc), wv[i].z), __fmul_rn(__fmul_rn(x[i].w, sc), wv[i].w));
         const float mx = max8(fmaxf(fmaxf(fabsf(y.x), fabsf(y.y)), fmaxf(fabsf(y.z), fabsf(y.w))));
         const float inv = mx > 0.f ? __fdiv_rn(127.f, mx) : 0.f;
         const int q0 = __float2int_rn(__fmul_rn(y.x, inv)), q1 = __float2int_rn(__fmul_rn(y.y, inv));
         const int q2 = __float2int_rn(__fmul_rn(y.z, inv)), q3 = __float2int_rn(__fmul_rn(y.w, inv));
-        if (own) {
+        if (e < n) {
             *reinterpret_cast<uint32_t*>(xq + bx_at(nb, t, e >> 5, e & 31)) =
                 (uint32_t)(q0 & 0xFF) | ((uint32_t)(q1 & 0xFF) << 8) | ((uint32_t)(q2 & 0xFF) << 16) | ((uint32_t)q3 << 24);
             if ((lane & 7) == 0) xd[bd_at(nb, t, e >> 5)] = f2h_bits(__fdiv_rn(mx, 127.f));
@@ -917,7 +929,7 @@ void launch_bulk(const DModel& M, const DLayer* layers, const BulkBuf& B, int p0
     const int E = M.E, ntt = (m + 63) / 64, nbE = E / 32;
     const int nsp = (p0 + m - 1) / (kAttnChunk * kAttnSplit) + 1;
     auto norm = [&](const float* w, const float* emb, int ks) {
-        LAUNCH(k_bnorm, (m + 3) / 4, kBThreads, s, E, M.eps, w, B.h, emb, M.tokbuf + p0, B.dpart, ks, m, B.xq, B.xd);
+        LAUNCH(k_bnorm, m, kBThreads, s, E, M.eps, w, B.h, emb, M.tokbuf + p0, B.dpart, ks, B.xq, B.xd);
     };
     int ks = 0;                                              // down partials the next norm adds
     for (int l = 0; l < M.NL; l++) {

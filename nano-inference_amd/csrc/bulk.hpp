@@ -9,9 +9,9 @@ namespace mi {
 constexpr int kBulkM = 2048;       // tokens of one panel, a multiple of 64. 1025 tokens in panels of 512 / 1024 /
                                    // 2048: 12.9 / 10.3 / 8.7 ms, 3001: 35.7 / 30.8 / 29.9 (1.5B shape): whole rounds
                                    // of workgroups and fewer launches
-// Shorter prompts stay with 8-token steps (1.4 ms each on the 1.5B shape, 0.98 on the 0.5B
-// one): a panel of 17 tokens takes 3.2 / 2.0 ms, three steps 4.2 / 2.9, two steps 2.8 / 2.0.
-constexpr int kBulkMin = 17;
+// Up to 8 tokens one multi-token step is faster: 1.41 ms on the 1.5B shape and 0.98 on the 0.5B
+// one against 1.95 and 1.20 for a panel; 9 tokens take a second step: 2.3 and 1.5.
+constexpr int kBulkMin = 9;
 constexpr int kBulkSplitM = 128;   // up to this many tokens the down GEMM runs one workgroup per K segment
 
 // Work buffers of a panel (device memory, kept by the engine). Int8 activations of an
