@@ -36,12 +36,6 @@ constexpr int kBThreads = 256;
 constexpr int kBulkWgs = 288;      // 9/8 of the 256 CUs
 constexpr int kKW = 8, kGThreads = 64 * kKW;   // waves of a GEMM workgroup: the chunks it runs at once
 
-// element offset of (token t, block b, element e of the block) in an operand buffer
-__host__ __device__ __forceinline__ size_t bx_at(int nb, int t, int b, int e) {
-    return ((((size_t)(t >> 5) * nb + b) * 64 + (e >> 4) * 32 + (t & 31)) << 4) + (e & 15);
-}
-__host__ __device__ __forceinline__ size_t bd_at(int nb, int t, int b) { return ((size_t)(t >> 5) * nb + b) * 32 + (t & 31); }
-
 BulkSizes bulk_sizes(int E, int FF, int NH, int HD, int QKV, int V, int maxseq, int ks_d) {
     const size_t M = kBulkM, nsp = (maxseq + kAttnChunk * kAttnSplit - 1) / (kAttnChunk * kAttnSplit);
     BulkSizes s;
@@ -455,20 +449,24 @@ __global__ __launch_bounds__(kBThreads, 2) void k_bgemm_w(PMat W, const int8_t* 
     }
 }
 
-// argmax and margin of token t (one wave): the candidates of its V/64 row groups
-__global__ __launch_bounds__(64) void k_bargmax(const float4* cand, int ng, int V, int t0, int p0, int32_t* out_tok,
-                                                float* out_margin) {
-    const int t = t0 + blockIdx.x, lane = threadIdx.x;
+// argmax and margin of one token: the candidates of its V/64 row groups (candidate row
+// blockIdx, position p0 + blockIdx); top-2 merging is associative and commutative
+__global__ __launch_bounds__(kBThreads) void k_bargmax(const float4* cand, int ng, int V, int p0, int32_t* out_tok,
+                                                       float* out_margin) {
+    __shared__ float4 wl[kBThreads / 64];
+    const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     Top2 a{-__builtin_inff(), INT_MAX, -__builtin_inff()};
-    for (int i = lane; i < ng; i += 64) {
+    for (int i = tid; i < ng; i += kBThreads) {
         const float4 c = cand[(size_t)t * ng + i];
         top2_merge(a, c.x, __float_as_int(c.y), c.z);
     }
     top2_wave(a);
-    if (lane == 0) {
-        out_tok[p0 + t] = top2_token(a, V);
-        out_margin[p0 + t] = __fsub_rn(a.best, a.second);
-    }
+    if (lane == 0) wl[tid >> 6] = make_float4(a.best, __int_as_float(a.idx), a.second, 0.f);
+    __syncthreads();
+    if (tid) return;
+    for (int w = 1; w < kBThreads / 64; w++) top2_merge(a, wl[w].x, __float_as_int(wl[w].y), wl[w].z);
+    out_tok[p0 + t] = top2_token(a, V);
+    out_margin[p0 + t] = __fsub_rn(a.best, a.second);
 }
 
 // ------------------------------------------------------------------ residual, norm, quant
@@ -962,11 +960,12 @@ void launch_bulk(const DModel& M, const DLayer* layers, const BulkBuf& B, int p0
     }
     if (!all && !last) return;
     norm(M.out_norm, nullptr, ks);
-    // predictions: every token tile, or only the one that holds the last token
-    const int tt0 = all ? 0 : ntt - 1, t0 = all ? 0 : m - 1;
-    gemm_w<BE_LM>(M.lm, B.xq + (size_t)(2 * tt0) * nbE * 1024, B.xd + (size_t)(2 * tt0) * nbE * 32, ntt - tt0, nullptr, nullptr,
-                  B.cand + (size_t)tt0 * 64 * (M.V / 64), s);
-    LAUNCH(k_bargmax, m - t0, 64, s, B.cand, M.V / 64, M.V, t0, p0, M.out_tok, M.out_margin);
+    // predictions of every token, or of the last one
+    if (all)
+        gemm_w<BE_LM>(M.lm, B.xq, B.xd, ntt, nullptr, nullptr, B.cand, s);
+    else
+        launch_lm_token(M.lm, B.xq, B.xd, m - 1, B.cand, s);
+    LAUNCH(k_bargmax, all ? m : 1, kBThreads, s, B.cand, M.V / 64, M.V, p0 + (all ? 0 : m - 1), M.out_tok, M.out_margin);
 }
 
 }  // namespace mi

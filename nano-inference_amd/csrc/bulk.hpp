@@ -29,6 +29,15 @@ struct BulkBuf {
     float* rec;                    // [kBulkM][NH][max splits][HD + 4] attention split records
     float4* cand;                  // [kBulkM][V/64] argmax candidates
 };
+// element offset of (token t, block b, element e of the block) in an operand buffer
+__host__ __device__ __forceinline__ size_t bx_at(int nb, int t, int b, int e) {
+    return ((((size_t)(t >> 5) * nb + b) * 64 + (e >> 4) * 32 + (t & 31)) << 4) + (e & 15);
+}
+__host__ __device__ __forceinline__ size_t bd_at(int nb, int t, int b) { return ((size_t)(t >> 5) * nb + b) * 32 + (t & 31); }
+
+// lm_head of token t of a panel (kernels.hip): V/64 argmax candidates
+void launch_lm_token(const PMat& W, const int8_t* xq, const uint32_t* xd, int t, float4* cand, hipStream_t s);
+
 struct BulkSizes { size_t h, xq, xd, qkv, aq, ad, dpart, rec, cand; };   // in elements
 BulkSizes bulk_sizes(int E, int FF, int NH, int HD, int QKV, int V, int maxseq, int ks_d);
 

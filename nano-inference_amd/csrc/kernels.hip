@@ -34,6 +34,7 @@
 // A wave's vector memory reads complete in issue order, so a prefetch issued by a
 // wave delays every later load of that same wave; keeping the barrier polls and the
 // prologue loads in a wave that never prefetches is what lets them overlap.
+#include "bulk.hpp"
 #include "common.hpp"
 #include "device.hpp"
 #include "kernels.hpp"
@@ -2642,6 +2643,44 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_wave(PMat W, const int8_t* xq,
         cur = nxt;
     }
     part[(size_t)s * W.rows + g * 64 + lane] = seg;
+}
+
+// lm_head of one token of a prompt panel (csrc/bulk.hip): a wave per 64-row group, the token's
+// codes from the panel's operand layout (bulk.hpp), each group's top-2 as an argmax candidate.
+// The panel's own GEMM would run 64 tokens for it: 87 us on the 1.5B shape.
+template <int CB>
+__global__ __launch_bounds__(kThreads) void k_lm_token(PMat W, const int8_t* xq, const uint32_t* xd, int t, float4* cand) {
+    __shared__ __align__(16) uint8_t X[(kMaxE / 32) * kXRec];
+    const int lane = threadIdx.x & 63, g = blockIdx.x * kWaves + (threadIdx.x >> 6), ng = W.rows >> 6;
+    for (int b = threadIdx.x; b < W.nb; b += kThreads) {
+        uint8_t* r = X + b * kXRec;
+        const int4 x0 = *reinterpret_cast<const int4*>(xq + bx_at(W.nb, t, b, 0));
+        const int4 x1 = *reinterpret_cast<const int4*>(xq + bx_at(W.nb, t, b, 16));
+        int sum = 0;
+        for (int v : {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w}) sum = __builtin_amdgcn_sdot4(v, 0x01010101, sum, false);
+        reinterpret_cast<int4*>(r)[0] = x0;
+        reinterpret_cast<int4*>(r)[1] = x1;
+        *reinterpret_cast<float*>(r + 32) = h2f_lo(xd[bd_at(W.nb, t, b)]);
+        *reinterpret_cast<int32_t*>(r + 36) = 8 * sum;
+    }
+    __syncthreads();
+    if (g >= ng) return;
+    float v = 0.f;
+    for (int c = 0; c < W.nc; c++) {
+        Tile tl;
+        tile_load_cb<CB>(tl, tile_ptr(W, g, c), lane);
+        const float p = chunk_dot<CB>(tl, X, kXRec, c * CB);
+        v = c ? __fadd_rn(v, p) : p;
+    }
+    Top2 a{-__builtin_inff(), INT_MAX, -__builtin_inff()};
+    top2_push(a, v, g * 64 + lane);
+    top2_wave(a);
+    if (lane == 0) cand[g] = make_float4(a.best, __int_as_float(a.idx), a.second, 0.f);
+}
+void launch_lm_token(const PMat& W, const int8_t* xq, const uint32_t* xd, int t, float4* cand, hipStream_t s) {
+    const int grid = ((W.rows >> 6) + kWaves - 1) / kWaves;
+    if (W.cb == 8) hipLaunchKernelGGL(k_lm_token<8>, dim3(grid), dim3(kThreads), 0, s, W, xq, xd, t, cand);
+    else hipLaunchKernelGGL(k_lm_token<4>, dim3(grid), dim3(kThreads), 0, s, W, xq, xd, t, cand);
 }
 
 __global__ void k_seg_sum(const float* part, int rows, int ks, float* y) {
