@@ -2506,9 +2506,12 @@ __global__ __launch_bounds__(kThreads) void k_quant(const float* x, int n, int8_
 // Otherwise four segments per workgroup, one chunk in flight per wave: the lower
 // register use keeps ~20 waves per CU resident, which is what feeds HBM for large
 // matrices.
+// y (may be null): one segment per row (ks = 1) is its own sum, so the kernel stores it as y
+// too and no k_seg_sum launch follows.
 constexpr int kGemvWgsPerCu = 2;
 template <bool SPREAD>
-__global__ __launch_bounds__(kThreads) void k_gemv(PMat W, const int8_t* xq, const float* xd, const int32_t* xs8, float* part) {
+__global__ __launch_bounds__(kThreads) void k_gemv(PMat W, const int8_t* xq, const float* xd, const int32_t* xs8, float* part,
+                                                   float* y) {
     __shared__ __align__(16) uint8_t X[(kMaxFF / 32) * kXRec];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int ntask = (W.rows / 64) * W.ks;
@@ -2536,6 +2539,7 @@ __global__ __launch_bounds__(kThreads) void k_gemv(PMat W, const int8_t* xq, con
                 seg = c == c0 ? p : __fadd_rn(seg, p);
             }
             part[(size_t)s * W.rows + g * 64 + lane] = seg;
+            if (y) y[g * 64 + lane] = seg;
         }
     } else {
         const int task = blockIdx.x;
@@ -2556,6 +2560,7 @@ __global__ __launch_bounds__(kThreads) void k_gemv(PMat W, const int8_t* xq, con
             cur = nxt;
         }
         part[(size_t)s * W.rows + g * 64 + lane] = seg;
+        if (y) y[g * 64 + lane] = seg;
     }
 }
 
@@ -2567,7 +2572,7 @@ __global__ __launch_bounds__(kThreads) void k_gemv(PMat W, const int8_t* xq, con
 constexpr int kSegMaxChunks = 48;
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void k_gemv_seg(PMat W, const int8_t* xq, const float* xd, const int32_t* xs8,
-                                                      float* part) {
+                                                      float* part, float* y) {
     __shared__ __align__(16) uint8_t X[kSegMaxChunks * 8 * kXRec];
     __shared__ float sums[kSegMaxChunks][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -2596,6 +2601,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_seg(PMat W, const int8_t* xq, 
         float seg = sums[0][lane];
         for (int k = 1; k < c1 - c0; k++) seg = __fadd_rn(seg, sums[k][lane]);
         part[(size_t)s * W.rows + g * 64 + lane] = seg;
+        if (y) y[g * 64 + lane] = seg;
     }
 }
 
@@ -2609,7 +2615,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_seg(PMat W, const int8_t* xq, 
 constexpr int kWaveMaxBlocks = 64;   // activation blocks of one wave's segment
 template <int NW, int CB>
 __global__ __launch_bounds__(64 * NW) void k_gemv_wave(PMat W, const int8_t* xq, const float* xd, const int32_t* xs8,
-                                                       float* part) {
+                                                       float* part, float* y) {
     __shared__ __align__(16) uint8_t X[NW][kWaveMaxBlocks * kXRec];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int task = blockIdx.x * NW + wave;
@@ -2643,6 +2649,53 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_wave(PMat W, const int8_t* xq,
         cur = nxt;
     }
     part[(size_t)s * W.rows + g * 64 + lane] = seg;
+    if (y) y[g * 64 + lane] = seg;
+}
+
+// Row-group-per-workgroup GEMV with its K segments summed in the same launch: wave j takes
+// chunks j, j + NW, ... of all of K (the next one's loads in flight), the chunk sums meet in
+// LDS, wave s adds segment s's (part), then wave 0 the segments (y): the orders of the
+// kernels above and k_seg_sum.
+// Taken for at most one workgroup per CU and up to 16 chunks per row; us per call from a graph
+// against segment kernel + k_seg_sum: 896 x 896 3.4 / 4.9, 2048 x 1536 3.8 / 5.4, 9728 x 896
+// 4.3 / 6.2, 7680 x 3840 (15 chunks) 7.9 / 9.8; past them 17920 x 1536 8.4 / 7.6, 896 x 4864
+// (19 chunks) 7.7 / 6.5, 1536 x 8960 (35) 10.8 / 7.4: too few CUs or waves share the stream.
+constexpr int kRowMaxGroups = 256, kRowMaxNc = 16;
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_gemv_row(PMat W, const int8_t* xq, const float* xd, const int32_t* xs8,
+                                                      float* part, float* y) {
+    __shared__ __align__(16) uint8_t X[kRowMaxNc * 8 * kXRec];
+    __shared__ float sums[kRowMaxNc][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = blockIdx.x;
+    Tile cur, nxt;
+    if (wave < W.nc) tile_load(cur, tile_ptr(W, g, wave), W.cb, lane);
+    for (int b = threadIdx.x; b < W.nb; b += 64 * NW) {
+        uint8_t* r = X + b * kXRec;
+        const uint4* src = reinterpret_cast<const uint4*>(xq + 32 * b);
+        reinterpret_cast<uint4*>(r)[0] = src[0];
+        reinterpret_cast<uint4*>(r)[1] = src[1];
+        *reinterpret_cast<float*>(r + 32) = xd[b];
+        *reinterpret_cast<int32_t*>(r + 36) = xs8[b];
+    }
+    __syncthreads();
+    for (int c = wave; c < W.nc; c += NW) {
+        if (c + NW < W.nc) tile_load(nxt, tile_ptr(W, g, c + NW), W.cb, lane);
+        sums[c][lane] = chunk_dot(cur, W.cb, X, kXRec, c * W.cb);
+        cur = nxt;
+    }
+    __syncthreads();
+    for (int s = wave; s < W.ks; s += NW) {                    // (a segment's sum replaces its first chunk's)
+        const int c0 = seg_c0(W, s);
+        const float v = seg_sum(&sums[0][0], c0, seg_c0(W, s + 1), lane);
+        part[(size_t)s * W.rows + g * 64 + lane] = v;
+        sums[c0][lane] = v;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        float v = sums[0][lane];
+        for (int s = 1; s < W.ks; s++) v = __fadd_rn(v, sums[seg_c0(W, s)][lane]);
+        y[g * 64 + lane] = v;
+    }
 }
 
 // lm_head of one token of a prompt panel (csrc/bulk.hip): a wave per 64-row group, the token's
@@ -3321,31 +3374,38 @@ void launch_quant(const float* x, int n, int8_t* xq, float* xd, int32_t* xs8, hi
 void launch_gemv(const PMat& W, const int8_t* xq, const float* xd, const int32_t* xs8, float* part, float* y,
                  int n_cu, hipStream_t s) {
     const int tasks = (W.rows / 64) * W.ks;
+    if (y && W.ks > 1 && W.rows / 64 <= kRowMaxGroups && W.nc <= kRowMaxNc) {
+        if (W.nc <= 4) LAUNCH(k_gemv_row<4>, W.rows / 64, 256, s, W, xq, xd, xs8, part, y);
+        else if (W.nc <= 8) LAUNCH(k_gemv_row<8>, W.rows / 64, 512, s, W, xq, xd, xs8, part, y);
+        else LAUNCH(k_gemv_row<12>, W.rows / 64, 768, s, W, xq, xd, xs8, part, y);
+        return;
+    }
+    float* y1 = W.ks == 1 ? y : nullptr;
     const int maxc = (W.nc + W.ks - 1) / W.ks;          // chunks of the longest segment
     const bool wave1 = maxc == 1, wave4 = tasks > kGemvWgsPerCu * n_cu && maxc * W.cb <= kWaveMaxBlocks;
     if (wave1 || wave4) {
         auto go = [&](auto cbv) {
             constexpr int CB = decltype(cbv)::value;
-            if (wave1) LAUNCH((k_gemv_wave<1, CB>), tasks, 64, s, W, xq, xd, xs8, part);
-            else LAUNCH((k_gemv_wave<4, CB>), (tasks + 3) / 4, 256, s, W, xq, xd, xs8, part);
+            if (wave1) LAUNCH((k_gemv_wave<1, CB>), tasks, 64, s, W, xq, xd, xs8, part, y1);
+            else LAUNCH((k_gemv_wave<4, CB>), (tasks + 3) / 4, 256, s, W, xq, xd, xs8, part, y1);
         };
         if (W.cb == 8) go(std::integral_constant<int, 8>());
         else go(std::integral_constant<int, 4>());
     } else if (tasks <= kGemvWgsPerCu * n_cu && maxc >= 2 && maxc <= kSegMaxChunks) {
         switch (std::min(maxc, 8)) {
-        case 2: LAUNCH(k_gemv_seg<2>, tasks, 128, s, W, xq, xd, xs8, part); break;
-        case 3: LAUNCH(k_gemv_seg<3>, tasks, 192, s, W, xq, xd, xs8, part); break;
-        case 4: LAUNCH(k_gemv_seg<4>, tasks, 256, s, W, xq, xd, xs8, part); break;
-        case 5: LAUNCH(k_gemv_seg<5>, tasks, 320, s, W, xq, xd, xs8, part); break;
-        case 6: LAUNCH(k_gemv_seg<6>, tasks, 384, s, W, xq, xd, xs8, part); break;
-        case 7: LAUNCH(k_gemv_seg<7>, tasks, 448, s, W, xq, xd, xs8, part); break;
-        default: LAUNCH(k_gemv_seg<8>, tasks, 512, s, W, xq, xd, xs8, part); break;
+        case 2: LAUNCH(k_gemv_seg<2>, tasks, 128, s, W, xq, xd, xs8, part, y1); break;
+        case 3: LAUNCH(k_gemv_seg<3>, tasks, 192, s, W, xq, xd, xs8, part, y1); break;
+        case 4: LAUNCH(k_gemv_seg<4>, tasks, 256, s, W, xq, xd, xs8, part, y1); break;
+        case 5: LAUNCH(k_gemv_seg<5>, tasks, 320, s, W, xq, xd, xs8, part, y1); break;
+        case 6: LAUNCH(k_gemv_seg<6>, tasks, 384, s, W, xq, xd, xs8, part, y1); break;
+        case 7: LAUNCH(k_gemv_seg<7>, tasks, 448, s, W, xq, xd, xs8, part, y1); break;
+        default: LAUNCH(k_gemv_seg<8>, tasks, 512, s, W, xq, xd, xs8, part, y1); break;
         }
     } else if (tasks <= kGemvWgsPerCu * n_cu)
-        LAUNCH(k_gemv<true>, tasks, kThreads, s, W, xq, xd, xs8, part);
+        LAUNCH(k_gemv<true>, tasks, kThreads, s, W, xq, xd, xs8, part, y1);
     else
-        LAUNCH(k_gemv<false>, std::min(4 * n_cu, (tasks + kWaves - 1) / kWaves), kThreads, s, W, xq, xd, xs8, part);
-    if (y) LAUNCH(k_seg_sum, (W.rows + 255) / 256, 256, s, part, W.rows, W.ks, y);
+        LAUNCH(k_gemv<false>, std::min(4 * n_cu, (tasks + kWaves - 1) / kWaves), kThreads, s, W, xq, xd, xs8, part, y1);
+    if (y && !y1) LAUNCH(k_seg_sum, (W.rows + 255) / 256, 256, s, part, W.rows, W.ks, y);
 }
 void launch_isums(const PMat& W, const int8_t* xq, int32_t* isum, hipStream_t s) {
     hipLaunchKernelGGL(k_isums, dim3(W.rows / 64, W.nb), dim3(64), 0, s, W, xq, isum);

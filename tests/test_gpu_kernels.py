@@ -84,6 +84,11 @@ GEMV_SHAPES = [  # (rows, in, cb, ks): S15 QKV/O/gate-up/down, S05 cb=4, lm_head
     (17920, 1536, 8, 6), (1536, 8960, 8, 10), (151936, 1536, 8, 2), (151936, 1536, 8, 1),
     (9728, 896, 4, 7),
 ]
+# row groups summed in the launch (ks > 1): one chunk per segment and fewer, 4 | 5, 8 | 9 and
+# 12 | 13 chunks (the workgroup sizes), 16 | 17 (the most), 256 | 257 row groups, the most segments
+GEMV_SHAPES += [(64, 64 * cb, cb, 2) for cb in (4, 8)] + [(128, 32 * 4 * nc, 4, ks) for nc, ks in (
+    (4, 3), (5, 5), (8, 2), (9, 4), (12, 12), (13, 6), (16, 16), (17, 17), (88, 88))]
+GEMV_SHAPES += [(64 * g, 512, 8, 2) for g in (256, 257)]
 
 
 @pytest.mark.parametrize("rows,n_in,cb,ks", GEMV_SHAPES)
