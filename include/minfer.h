@@ -264,7 +264,7 @@ int mi_q4_block_isums(const uint8_t* packed, int32_t rows, int32_t nb, int32_t c
 
 /* single-query GQA attention over an fp16 cache (cuda_infer.cu:650-702 attn_partial +
  * attn_combine, mega.cu:414-521), two kernel launches on `stream` (chunk records, then
- * their merge): q[n_head][hd] fp32, kc/vc [n_head_kv][ctx][hd] fp16, positions 0..L-1,
+ * their merge), or one up to 512 positions: q[n_head][hd] fp32, kc/vc [n_head_kv][ctx][hd] fp16, positions 0..L-1,
  * out[n_head][hd]; n_head / n_head_kv <= 8, at most 512 splits of 16 64-position chunks
  * (L <= 524288). scratch holds mi_attn_scratch_floats(n_head, hd, L) floats: a record
  * per head and 64-position chunk, written and read within the call (no initial

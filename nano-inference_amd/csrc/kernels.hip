@@ -2842,6 +2842,103 @@ __global__ __launch_bounds__(64 * (S * ((kAttnMaxG + H - 1) / H) + 1)) void k_at
     }
 }
 
+// Standalone attention of a short context in one launch: one workgroup per query head, wave c
+// on chunk c (up to kOneChunks). K comes by DMA into the wave's swizzled tile; V is not shared between waves, so a lane loads its dims of all 64 rows
+// straight into registers, everything in flight at once. The chunk arithmetic is
+// attn_core_h's, the merge the canonical one of up to 16 chunks. The query heads of a kv head
+// read its rows from the L2. us per call from a graph, one launch / k_attn_rec + k_attn_merge /
+// k_attn_mx + k_attn_merge: hd 128 at 64 positions 5.2 / 7.8 / 6.9, 256 6.0 / 8.1 / 7.1, 512 8.2 /
+// 8.3 / 7.3; hd 64 at 512 6.1 / 7.5 / 6.5, 1024 (16 waves on one CU) 10.0 / 7.6 / 6.6. Called
+// eagerly it saves the second launch: 9.5 against 12.2.
+constexpr int kOneChunks = 8, kOneChunksMx128 = 4;            // (against k_attn_mx at hd 128)
+template <int HD>
+__device__ __forceinline__ void one_issue_k(const __half* krows, int n, uint8_t* tile, int lane) {
+    constexpr int NV = HD / 8, RPI = 64 / NV;
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int t = i * RPI + lane / NV;
+        const __half* src = krows + (size_t)min(t, n - 1) * HD + 8 * ((lane % NV) ^ kswz<HD>(t));
+        __builtin_amdgcn_global_load_lds(src, (lds_ptr)(tile + i * 1024), 16, 0, 0);
+    }
+}
+template <int HD, int NW>
+__global__ __launch_bounds__(64 * NW) void k_attn_one(const float* q, const __half* kc, const __half* vc, int G, int L, int ctx,
+                                                      float scale, float* out) {
+    constexpr int NV = HD / 8, DPL = HD / 64;
+    __shared__ __align__(16) uint8_t kt[NW][64 * HD * 2];
+    __shared__ __align__(16) float qs[HD], pl[NW][64], ol[NW][HD];
+    __shared__ float ml[NW], ll[NW];
+    const int lane = threadIdx.x & 63, c = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = blockIdx.x;
+    const int nch = (L + kAttnChunk - 1) / kAttnChunk, t0 = c * kAttnChunk, n = min(kAttnChunk, L - t0);
+    using VT = typename std::conditional<DPL == 2, uint32_t, uint16_t>::type;
+    VT vr[64];
+    for (int i = threadIdx.x; i < HD; i += 64 * NW) qs[i] = q[h * HD + i];
+    if (c < nch) {
+        const size_t row = (size_t)(h / G) * ctx + t0;
+        one_issue_k<HD>(kc + row * HD, n, kt[c], lane);
+        const __half* v = vc + row * HD + DPL * lane;
+#pragma unroll
+        for (int t = 0; t < 64; t++) vr[t] = *reinterpret_cast<const VT*>(v + (size_t)min(t, n - 1) * HD);
+        drain_vm();
+    }
+    __syncthreads();
+    if (c < nch) {
+        const uint4* kls = reinterpret_cast<const uint4*>(kt[c]);
+        float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+#pragma unroll 4
+        for (int j = 0; j < NV; j++) {
+            const uint4 w = kls[kslot<HD>(lane, j)];
+            const float4 q0 = ld4(qs + 8 * j), q1 = ld4(qs + 8 * j + 4);
+            a0 = __fmaf_rn(q0.x, h2f_lo(w.x), a0); a1 = __fmaf_rn(q0.y, h2f_hi(w.x), a1);
+            a2 = __fmaf_rn(q0.z, h2f_lo(w.y), a2); a3 = __fmaf_rn(q0.w, h2f_hi(w.y), a3);
+            a0 = __fmaf_rn(q1.x, h2f_lo(w.z), a0); a1 = __fmaf_rn(q1.y, h2f_hi(w.z), a1);
+            a2 = __fmaf_rn(q1.z, h2f_lo(w.w), a2); a3 = __fmaf_rn(q1.w, h2f_hi(w.w), a3);
+        }
+        const bool valid = lane < n;
+        const float s = valid ? __fmul_rn(__fadd_rn(__fadd_rn(a0, a1), __fadd_rn(a2, a3)), scale) : -__builtin_inff();
+        const float m = wave_max(s);
+        const float p = valid ? mi_expf(__fsub_rn(s, m)) : 0.f;
+        const float ls = bfly_sum64(p);
+        pl[c][lane] = p;
+        wave_lds_sync();
+        float acc[DPL];
+#pragma unroll
+        for (int e = 0; e < DPL; e++) acc[e] = 0.f;
+        const int ns = __builtin_amdgcn_readfirstlane(n);
+#pragma unroll
+        for (int t4 = 0; t4 < 16; t4++) {
+            const float4 pv = ld4(&pl[c][4 * t4]);
+            const float pt[4] = {pv.x, pv.y, pv.z, pv.w};
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (4 * t4 + u < ns) {                       // positions past n are not part of the chain
+                    if constexpr (DPL == 2) {
+                        acc[0] = __fmaf_rn(pt[u], h2f_lo(vr[4 * t4 + u]), acc[0]);
+                        acc[1] = __fmaf_rn(pt[u], h2f_hi(vr[4 * t4 + u]), acc[1]);
+                    } else {
+                        acc[0] = __fmaf_rn(pt[u], __half2float(__ushort_as_half(vr[4 * t4 + u])), acc[0]);
+                    }
+                }
+        }
+#pragma unroll
+        for (int e = 0; e < DPL; e++) ol[c][DPL * lane + e] = acc[e];
+        if (lane == 0) { ml[c] = m; ll[c] = ls; }
+    }
+    __syncthreads();
+    const int d = threadIdx.x;
+    if (d < HD) {
+        float M = ml[0];
+        for (int i = 1; i < nch; i++) M = fmaxf(M, ml[i]);
+        float den = 0.f, o = 0.f;
+        for (int i = 0; i < nch; i++) {
+            const float w = mi_expf(__fsub_rn(ml[i], M));
+            den = __fmaf_rn(ll[i], w, den);
+            o = __fmaf_rn(ol[i][d], w, o);
+        }
+        out[h * HD + d] = __fdiv_rn(o, den);
+    }
+}
+
 // Standalone attention, part 2: the canonical merge (orc_attention_canon's order, the
 // step's merge phase's) of one head's chunk records, for 32 of its dims (one 128-byte
 // line of each o record) per workgroup. Wave w takes the split pairs (2g, 2g + 1) for
@@ -3432,11 +3529,26 @@ static void launch_attn_rec(const float* q, const __half* kc, const __half* vc, 
     const int grid = min((units + S - 1) / S, device_cus() * per_cu);
     LAUNCH((k_attn_rec<HD, H, S>), grid, 64 * (S * ((G + H - 1) / H) + 1), s, q, kc, vc, nh, nkv, L, ctx, scale, recs);
 }
+// up to maxch chunks: one launch instead of two
+static bool launch_attn_one(const float* q, const __half* kc, const __half* vc, int nh, int nkv, int hd, int nch, int maxch, int L,
+                            int ctx, float scale, float* out, hipStream_t s) {
+    if (nch > maxch) return false;
+    const int G = nh / nkv;
+    with_hd(hd, [&](auto hc) {
+        constexpr int HD = decltype(hc)::value;
+        // at least HD threads: the merge is a thread per dim
+        if (nch <= 2) LAUNCH((k_attn_one<HD, 2>), nh, 128, s, q, kc, vc, G, L, ctx, scale, out);
+        else if (nch <= 4) LAUNCH((k_attn_one<HD, 4>), nh, 256, s, q, kc, vc, G, L, ctx, scale, out);
+        else LAUNCH((k_attn_one<HD, 8>), nh, 512, s, q, kc, vc, G, L, ctx, scale, out);
+    });
+    return true;
+}
 bool launch_attn_decode(const float* q, const __half* kc, const __half* vc, int nh, int nkv, int hd, int L, int ctx,
                         float scale, float* scratch, float* out, hipStream_t s) {
     if (nh % nkv || !kernels_support(nh / nkv, hd) || nh / nkv > kAttnMaxG || L < 1) return false;
     const int nch = (L + kAttnChunk - 1) / kAttnChunk, nsp = (nch + kAttnSplit - 1) / kAttnSplit;
     if (nsp > kAttnMaxSplits) return false;
+    if (launch_attn_one(q, kc, vc, nh, nkv, hd, nch, kOneChunks, L, ctx, scale, out, s)) return true;
     with_hd(hd, [&](auto h) {
         constexpr int HD = decltype(h)::value;
         // one head per compute wave, one unit per round (two workgroups per CU at hd 128):
@@ -3454,6 +3566,7 @@ bool launch_attn_decode_mfma(const float* q, const __half* kc, const __half* vc,
     if (nh % nkv || !kernels_support(nh / nkv, hd) || nh / nkv > kAttnMaxG || L < 1) return false;
     const int nch = (L + kAttnChunk - 1) / kAttnChunk, nsp = (nch + kAttnSplit - 1) / kAttnSplit;
     if (nsp > kAttnMaxSplits) return false;
+    if (launch_attn_one(q, kc, vc, nh, nkv, hd, nch, hd == 128 ? kOneChunksMx128 : kOneChunks, L, ctx, scale, out, s)) return true;
     with_hd(hd, [&](auto h) {
         constexpr int HD = decltype(h)::value;
         const int units = nkv * nch, per_cu = max(1, (160 * 1024) / amx_lds<HD>());

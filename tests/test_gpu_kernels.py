@@ -112,6 +112,11 @@ def test_gemv_bit_exact(torch, rows, n_in, cb, ks):
 @pytest.mark.parametrize("nh,nkv,hd,L", [(12, 2, 128, 1), (12, 2, 128, 64), (12, 2, 128, 65), (12, 2, 128, 300),
                                          (14, 2, 64, 200), (16, 2, 128, 1024), (4, 2, 64, 130),
                                          (14, 2, 64, 1100), (16, 2, 128, 2049), (8, 1, 128, 5000),
+                                         # one launch up to 8 chunks: its 2, 4 and 8-wave forms
+                                         # and the first past them
+                                         (12, 2, 128, 128), (12, 2, 128, 129), (16, 2, 128, 257), (8, 1, 128, 512),
+                                         (12, 2, 128, 513), (14, 2, 64, 1), (14, 2, 64, 63), (3, 3, 64, 512),
+                                         (14, 2, 64, 513),
                                          (32, 4, 64, 32768), (24, 4, 128, 32700), (12, 2, 128, 33000)])
 def test_attention_bit_exact(torch, nh, nkv, hd, L):
     """chunked attention vs the oracle's canonical order; the last three cases give
