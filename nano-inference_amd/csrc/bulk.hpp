@@ -12,7 +12,11 @@ constexpr int kBulkM = 2048;       // tokens of one panel, a multiple of 64. 102
 // Up to 8 tokens one multi-token step is faster: 1.41 ms on the 1.5B shape and 0.98 on the 0.5B
 // one against 1.95 and 1.20 for a panel; 9 tokens take a second step: 2.3 and 1.5.
 constexpr int kBulkMin = 9;
-constexpr int kBulkSplitM = 128;   // up to this many tokens the down GEMM runs one workgroup per K segment
+// Up to this many tokens the down GEMM runs one workgroup per K segment: its 64 x 64 tiles alone
+// are too few for the CUs. Whole prefill, split / not, ms: 1.5B shape 129 tokens 2.85 / 3.24,
+// 256 3.16 / 3.37, 257 3.56 / 3.62, 321 3.85 / 3.73, 512 4.85 / 4.36; 0.5B shape 1.69 / 1.74,
+// 1.76 / 1.80, 1.94 / 1.85, 2.13 / 1.93, 2.62 / 2.28.
+constexpr int kBulkSplitM = 256;
 
 // Work buffers of a panel (device memory, kept by the engine). Int8 activations of an
 // nb-block vector per token are stored as the GEMM's MFMA operand: 32-token tiles, per tile

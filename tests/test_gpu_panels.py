@@ -4,7 +4,7 @@ per 7 tokens (tchunk=7, itself bit-identical to single steps and the q8act oracl
 predictions, the margins and, through a step's logits, the K/V the panel left.
 
 Lengths sit on the edges of the 32-token tiles, the 64-token GEMM tiles, the panel whose down
-matrix is split over workgroups (128), the attention split (1024) and the panel (2048)."""
+matrix is split over workgroups (256), the attention split (1024) and the panel (2048)."""
 import sys
 
 import numpy as np
@@ -42,7 +42,7 @@ def pair(request):
     b.close()
 
 
-@pytest.mark.parametrize("n", [9, 17, 32, 33, 63, 64, 65, 128, 129, 257, 512, 513, 1024, 1025, 1151, 2048, 2049])
+@pytest.mark.parametrize("n", [9, 17, 32, 33, 63, 64, 65, 128, 129, 256, 257, 512, 513, 1024, 1025, 1151, 2048, 2049])
 def test_panel_bit_identical(pair, n):
     shape, a, b = pair
     print("[gpu-panel] n", n, flush=True)
