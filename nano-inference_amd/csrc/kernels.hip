@@ -2845,12 +2845,10 @@ __global__ __launch_bounds__(64 * (S * ((kAttnMaxG + H - 1) / H) + 1)) void k_at
 // Standalone attention of a short context in one launch: one workgroup per query head, wave c
 // on chunk c (up to kOneChunks). K comes by DMA into the wave's swizzled tile; V is not shared between waves, so a lane loads its dims of all 64 rows
 // straight into registers, everything in flight at once. The chunk arithmetic is
-// attn_core_h's, the merge the canonical one of up to 16 chunks. The query heads of a kv head
-// read its rows from the L2. us per call from a graph, one launch / k_attn_rec + k_attn_merge /
-// k_attn_mx + k_attn_merge: hd 128 at 64 positions 5.2 / 7.8 / 6.9, 256 6.0 / 8.1 / 7.1, 512 8.2 /
-// 8.3 / 7.3; hd 64 at 512 6.1 / 7.5 / 6.5, 1024 (16 waves on one CU) 10.0 / 7.6 / 6.6. Called
-// eagerly it saves the second launch: 9.5 against 12.2.
+// attn_core_h's, the merge the canonical one of up to kOneChunks chunks. The query heads of a kv
+// head read its rows from the L2 (which calls take it, and the times: attn_one_takes).
 constexpr int kOneChunks = 8, kOneChunksMx128 = 4;            // (against k_attn_mx at hd 128)
+constexpr int kOneHeadDims = 131072;
 template <int HD>
 __device__ __forceinline__ void one_issue_k(const __half* krows, int n, uint8_t* tile, int lane) {
     constexpr int NV = HD / 8, RPI = 64 / NV;
@@ -3529,11 +3527,27 @@ static void launch_attn_rec(const float* q, const __half* kc, const __half* vc, 
     const int grid = min((units + S - 1) / S, device_cus() * per_cu);
     LAUNCH((k_attn_rec<HD, H, S>), grid, 64 * (S * ((G + H - 1) / H) + 1), s, q, kc, vc, nh, nkv, L, ctx, scale, recs);
 }
-// up to maxch chunks: one launch instead of two
-static bool launch_attn_one(const float* q, const __half* kc, const __half* vc, int nh, int nkv, int hd, int nch, int maxch, int L,
+// The calls k_attn_one takes (mx: mi_attn_decode_mfma's). us per call from a graph, k_attn_one /
+// k_attn_rec + k_attn_merge / k_attn_mx + k_attn_merge:
+//   12/2 heads, hd 128: 64 positions 5.3 / 8.0 / 7.0, 256 6.1 / 8.1 / 7.1, 512 7.9 / 8.3 / 7.3
+//   14/2 heads, hd 64:  64 positions 4.0 / 6.8 / 5.9, 512 6.1 / 7.5 / 6.6; 1024 positions (16 waves on
+//                       one CU) 10.0 / 7.6 / 6.6
+// Its workgroups read a kv head's rows once per query head, the other two kernels once or twice:
+// past about 32 MiB of such reads (kOneHeadDims: heads x chunks x dims) the L2 holds it up.
+// 32 kv heads of 8 at hd 128: 256 positions (at the line) 6.8 / 10.9 / 9.7, 320 11.8 / 11.1, 512 15.2 /
+// 11.6; 48 of 8 at hd 64: 320 (under it) 6.7 / 9.9 / 8.7, 384 (past it) 10.1 / 11.1 / 9.1, 512 12.8 / 11.5 /
+// 9.5. Without sharing (G = 1) there is nothing to lose: 512 heads of 64 at 512 positions 14.6 /
+// 18.0 / 19.2. The eighth chunk at hd 128 loses to k_attn_rec's two heads per unit (G = 2, 48 kv
+// heads: 9.8 / 8.5) and to its single ones while they leave CUs idle (8/8 7.8 / 7.6, 96/96 the other way).
+static bool attn_one_takes(int nh, int G, int hd, int nch, bool mx) {
+    if (nch > (mx && hd == 128 ? kOneChunksMx128 : kOneChunks)) return false;
+    if (hd == 128 && nch == kOneChunks && (G == 2 || (G == 1 && nh <= 64))) return false;
+    return G == 1 || (int64_t)nh * nch * hd <= kOneHeadDims;
+}
+static bool launch_attn_one(const float* q, const __half* kc, const __half* vc, int nh, int nkv, int hd, int nch, bool mx, int L,
                             int ctx, float scale, float* out, hipStream_t s) {
-    if (nch > maxch) return false;
     const int G = nh / nkv;
+    if (!attn_one_takes(nh, G, hd, nch, mx)) return false;
     with_hd(hd, [&](auto hc) {
         constexpr int HD = decltype(hc)::value;
         // at least HD threads: the merge is a thread per dim
@@ -3548,7 +3562,7 @@ bool launch_attn_decode(const float* q, const __half* kc, const __half* vc, int 
     if (nh % nkv || !kernels_support(nh / nkv, hd) || nh / nkv > kAttnMaxG || L < 1) return false;
     const int nch = (L + kAttnChunk - 1) / kAttnChunk, nsp = (nch + kAttnSplit - 1) / kAttnSplit;
     if (nsp > kAttnMaxSplits) return false;
-    if (launch_attn_one(q, kc, vc, nh, nkv, hd, nch, kOneChunks, L, ctx, scale, out, s)) return true;
+    if (launch_attn_one(q, kc, vc, nh, nkv, hd, nch, false, L, ctx, scale, out, s)) return true;
     with_hd(hd, [&](auto h) {
         constexpr int HD = decltype(h)::value;
         // one head per compute wave, one unit per round (two workgroups per CU at hd 128):
@@ -3566,7 +3580,7 @@ bool launch_attn_decode_mfma(const float* q, const __half* kc, const __half* vc,
     if (nh % nkv || !kernels_support(nh / nkv, hd) || nh / nkv > kAttnMaxG || L < 1) return false;
     const int nch = (L + kAttnChunk - 1) / kAttnChunk, nsp = (nch + kAttnSplit - 1) / kAttnSplit;
     if (nsp > kAttnMaxSplits) return false;
-    if (launch_attn_one(q, kc, vc, nh, nkv, hd, nch, hd == 128 ? kOneChunksMx128 : kOneChunks, L, ctx, scale, out, s)) return true;
+    if (launch_attn_one(q, kc, vc, nh, nkv, hd, nch, true, L, ctx, scale, out, s)) return true;
     with_hd(hd, [&](auto h) {
         constexpr int HD = decltype(h)::value;
         const int units = nkv * nch, per_cu = max(1, (160 * 1024) / amx_lds<HD>());

@@ -142,6 +142,43 @@ def test_attention_bit_exact(torch, nh, nkv, hd, L):
         assert np.array_equal(got[h].view(np.uint32), ref.view(np.uint32)), h
 
 
+@pytest.mark.parametrize("mfma", [False, True], ids=["canon", "mfma"])
+@pytest.mark.parametrize("nh,nkv,hd,L,one", [
+    # heads x chunks x head size on either side of 131072
+    (256, 32, 128, 256, (1, 1)), (256, 32, 128, 257, (0, 0)), (257, 257, 128, 256, (1, 1)), (160, 20, 128, 448, (0, 0)),
+    (256, 32, 64, 512, (1, 1)), (264, 33, 64, 512, (0, 0)), (512, 64, 64, 256, (1, 1)), (512, 64, 64, 257, (0, 0)),
+    # the eighth chunk at head size 128
+    (4, 2, 128, 448, (1, 0)), (4, 2, 128, 449, (0, 0)), (8, 8, 128, 449, (0, 0)), (65, 65, 128, 449, (1, 0)),
+    (12, 2, 128, 512, (1, 0)), (12, 2, 128, 513, (0, 0)), (14, 2, 64, 512, (1, 1)), (14, 2, 64, 513, (0, 0))])
+def test_attention_one_launch_lines(torch, nh, nkv, hd, L, one, mfma):
+    """both sides of the lines between one launch and chunk records + merge: which side runs
+    shows in the scratch (one launch writes none), the values against the canonical order
+    (bit for bit, except the matrix-core records: 1e-5, see test_gpu_attn_mfma.py)"""
+    one = bool(one[mfma])
+    say("attention line nh=%d nkv=%d hd=%d L=%d mfma=%d" % (nh, nkv, hd, L, mfma))
+    rng = np.random.default_rng(nh + L)
+    q = rng.standard_normal((nh, hd)).astype(np.float32)
+    k16 = rng.standard_normal((nkv, L, hd)).astype(np.float16)
+    v16 = rng.standard_normal((nkv, L, hd)).astype(np.float16)
+    scale = np.float32(1.0) / np.float32(math.sqrt(hd))
+    scratch = torch.full((minfer.attn_scratch_floats(nh, hd, L),), float("nan"), device="cuda")
+    out = torch.zeros(nh * hd, device="cuda")
+    fn = minfer.attn_decode_mfma if mfma else minfer.attn_decode
+    fn(dev(torch, q), dev(torch, k16.view(np.int16)), dev(torch, v16.view(np.int16)), nh, nkv, hd, L, L, float(scale),
+       scratch, out)
+    torch.cuda.synchronize()
+    assert bool(torch.isnan(scratch).all()) == one
+    got = out.cpu().numpy().reshape(nh, hd)
+    G = nh // nkv
+    for h in sorted({0, nh // 3, nh // 2, nh - 1}):
+        kf = np.ascontiguousarray(k16[h // G].astype(np.float32))
+        vf = np.ascontiguousarray(v16[h // G].astype(np.float32))
+        ref = O.attention_canon(np.ascontiguousarray(q[h]), kf.ravel(), vf.ravel(), L, hd, hd, float(scale))
+        if mfma and not one:
+            assert np.abs(got[h] - ref).max() <= 1e-5 * np.abs(ref).max(), h
+        else:
+            assert np.array_equal(got[h].view(np.uint32), ref.view(np.uint32)), h
+
 def test_stream_read_runs(torch):
     say("stream read 256 MB")
     buf = torch.zeros(256 << 20, dtype=torch.uint8, device="cuda")
