@@ -2656,10 +2656,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_wave(PMat W, const int8_t* xq,
 // chunks j, j + NW, ... of all of K (the next one's loads in flight), the chunk sums meet in
 // LDS, wave s adds segment s's (part), then wave 0 the segments (y): the orders of the
 // kernels above and k_seg_sum.
-// Taken for at most one workgroup per CU and up to 16 chunks per row; us per call from a graph
-// against segment kernel + k_seg_sum: 896 x 896 3.4 / 4.9, 2048 x 1536 3.8 / 5.4, 9728 x 896
-// 4.3 / 6.2, 7680 x 3840 (15 chunks) 7.9 / 9.8; past them 17920 x 1536 8.4 / 7.6, 896 x 4864
-// (19 chunks) 7.7 / 6.5, 1536 x 8960 (35) 10.8 / 7.4: too few CUs or waves share the stream.
+// (which calls take it: gemv_row_takes)
 constexpr int kRowMaxGroups = 256, kRowMaxNc = 16;
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void k_gemv_row(PMat W, const int8_t* xq, const float* xd, const int32_t* xs8,
@@ -3458,6 +3455,20 @@ int persistent_max_grid(int G, int HD) {
 void launch_quant(const float* x, int n, int8_t* xq, float* xd, int32_t* xs8, hipStream_t s) {
     LAUNCH(k_quant, (n + kThreads - 1) / kThreads, kThreads, s, x, n, xq, xd, xs8);
 }
+// The calls k_gemv_row takes; us per call from a graph, it / segment kernel + k_seg_sum.
+// At most one workgroup per CU and 16 chunks per row: 896 x 896 3.4 / 4.9, 2048 x 1536 3.8 / 5.4,
+// 9728 x 896 4.3 / 6.2, 7680 x 3840 (15 chunks of 4 blocks) 7.9 / 9.8; past them 17920 x 1536 8.4 / 7.6,
+// 896 x 4864 (19 chunks) 7.7 / 6.5, 1536 x 8960 (35) 10.8 / 7.4: too few CUs or waves share the stream.
+// Rows of more than 88 blocks (11 chunks of 8) stay with the segment kernel while a workgroup per
+// segment spreads them wider: up to 128 row groups, 512 segments in all and 10 per row. 3072 rows in 4
+// segments: 88 blocks 5.5 / 5.5, 96 5.7 / 5.5, 104 6.4 / 5.5, 128 6.8 / 5.6; 128 blocks on the other side of each line:
+// 10240 rows in 2 segments 7.5 / 10.1, 6144 in 10 7.3 / 8.0, 3072 in 11 7.2 / 7.8.
+constexpr int kRowFreeBlocks = 88, kRowGroups = 128, kRowTasks = 512, kRowKs = 10;
+static bool gemv_row_takes(const PMat& W) {
+    const int ng = W.rows / 64;
+    if (ng > kRowMaxGroups || W.nc > kRowMaxNc) return false;
+    return W.nb <= kRowFreeBlocks || ng > kRowGroups || ng * W.ks > kRowTasks || W.ks > kRowKs;
+}
 // Kernel choice by segment count and length (sweep on the box, config-1 shapes, µs per
 // launch from graph replay; every choice gives the same bits):
 // * one-chunk segments (qkv, o, gate/up at ks 6): one wave per segment, 1-wave workgroups
@@ -3469,7 +3480,7 @@ void launch_quant(const float* x, int n, int8_t* xq, float* xd, int32_t* xs8, hi
 void launch_gemv(const PMat& W, const int8_t* xq, const float* xd, const int32_t* xs8, float* part, float* y,
                  int n_cu, hipStream_t s) {
     const int tasks = (W.rows / 64) * W.ks;
-    if (y && W.ks > 1 && W.rows / 64 <= kRowMaxGroups && W.nc <= kRowMaxNc) {
+    if (y && W.ks > 1 && gemv_row_takes(W)) {
         if (W.nc <= 4) LAUNCH(k_gemv_row<4>, W.rows / 64, 256, s, W, xq, xd, xs8, part, y);
         else if (W.nc <= 8) LAUNCH(k_gemv_row<8>, W.rows / 64, 512, s, W, xq, xd, xs8, part, y);
         else LAUNCH(k_gemv_row<12>, W.rows / 64, 768, s, W, xq, xd, xs8, part, y);

@@ -89,6 +89,9 @@ GEMV_SHAPES = [  # (rows, in, cb, ks): S15 QKV/O/gate-up/down, S05 cb=4, lm_head
 GEMV_SHAPES += [(64, 64 * cb, cb, 2) for cb in (4, 8)] + [(128, 32 * 4 * nc, 4, ks) for nc, ks in (
     (4, 3), (5, 5), (8, 2), (9, 4), (12, 12), (13, 6), (16, 16), (17, 17), (88, 88))]
 GEMV_SHAPES += [(64 * g, 512, 8, 2) for g in (256, 257)]
+# long rows: 88 | 96 blocks, 128 | 129 row groups, 512 | 520 segments in all, 10 | 11 segments per row
+GEMV_SHAPES += [(1024, 32 * 88, 8, 4), (1024, 32 * 96, 8, 4), (8192, 3072, 8, 2), (8256, 3072, 8, 2), (4096, 3072, 8, 8),
+                (4160, 3072, 8, 8), (320, 4096, 8, 10), (320, 4096, 8, 11)]
 
 
 @pytest.mark.parametrize("rows,n_in,cb,ks", GEMV_SHAPES)
