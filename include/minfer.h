@@ -41,7 +41,11 @@ typedef struct mi_opts {
     int32_t max_ctx;       /* KV cache capacity in positions (0: 4096) */
     int32_t tchunk;        /* prompt tokens per step, 1..8. At 8 (the default) prompts of 9 tokens and more
                               take panels of up to 2048 tokens per pass over the weights instead (same
-                              bits; 512 tokens of the 1.5B shape: 84.1 -> 4.5 ms) */
+                              bits; 512 tokens of the 1.5B shape: 84.1 -> 4.5 ms). The panels' work buffers
+                              are part of the engine: 120 / 149 / 162 MB on the 0.5B / 1.5B / 3B shape at
+                              max_ctx 4352, 123 / 272 / 349 at 32768, 8 MB at 64, none at tchunk < 8 or
+                              max_ctx < 9. Where mi_load finds no memory for them the prompts run
+                              in steps of 8 */
     int32_t spec;          /* n-gram speculative decoding inside mi_generate: 0 off; 1 the host drafts,
                               launches each verify step and commits its result; 2 the whole loop runs
                               on the device (mega.cu:863-895: each persistent verify launch commits
@@ -230,7 +234,8 @@ int mi_synth_gguf(const char* path, const mi_synth_shape* shape, uint64_t seed);
  * counterpart in the reference: for a model shape, a context of max_ctx positions and a
  * grid of n_cu workgroups, walks every index the single-token step (T = 1) or the
  * multi-token phase bodies (T = 2..8) form for a step at pos, with each body's loop
- * bounds, against the allocation sizes the engine uses. Returns MI_OK, MI_ERR_SHAPE with
+ * bounds, against the allocation sizes the engine uses, and the ends of what a prompt of
+ * pos + T tokens reads and writes in panels. Returns MI_OK, MI_ERR_SHAPE with
  * the buffer and index in err, or MI_ERR_ARG. */
 int mi_check_layout(const mi_synth_shape* shape, int32_t max_ctx, int32_t n_cu, int32_t T, int32_t pos, char* err,
                     int32_t errlen);

@@ -36,8 +36,14 @@ constexpr int kBThreads = 256;
 constexpr int kBulkWgs = 288;      // 9/8 of the 256 CUs
 constexpr int kKW = 8, kGThreads = 64 * kKW;   // waves of a GEMM workgroup: the chunks it runs at once
 
-BulkSizes bulk_sizes(int E, int FF, int NH, int HD, int QKV, int V, int maxseq, int ks_d) {
-    const size_t M = kBulkM, nsp = (maxseq + kAttnChunk * kAttnSplit - 1) / (kAttnChunk * kAttnSplit);
+static size_t rec_floats(int NH, int HD, int nsp) { return (size_t)NH * nsp * (HD + 4); }   // of one token
+
+static size_t pad256(size_t n) { return (n + 255) & ~size_t(255); }
+
+BulkSizes bulk_sizes(int E, int FF, int NH, int HD, int QKV, int V, int maxseq, int ks_d, size_t kv) {
+    const size_t M = std::min(kBulkM, (maxseq + 63) / 64 * 64);
+    const int nsp = (maxseq + kAttnChunk * kAttnSplit - 1) / (kAttnChunk * kAttnSplit);
+    const size_t tok = nsp > 1 ? rec_floats(NH, HD, nsp) : 0;
     BulkSizes s;
     s.h = M * E;
     s.xq = M * E;
@@ -45,10 +51,41 @@ BulkSizes bulk_sizes(int E, int FF, int NH, int HD, int QKV, int V, int maxseq, 
     s.qkv = M * QKV;
     s.aq = M * FF;
     s.ad = M * (FF / 32);
-    s.dpart = (size_t)ks_d * kBulkSplitM * E;
-    s.rec = M * NH * nsp * (HD + 4);
+    s.dpart = (size_t)ks_d * std::min<size_t>(kBulkSplitM, M) * E;
     s.cand = M * (V / 64);
+    const size_t idle = pad256(s.aq) + pad256(4 * s.ad) + pad256(4 * s.dpart) + pad256(16 * s.cand);
+    s.rec = std::max(idle / 4, std::min(M * tok, std::max(std::max(kBulkRecFloats, kv / 4), 32 * tok)));
     return s;
+}
+
+size_t bulk_bind(const BulkSizes& s, void* base, BulkBuf* B) {
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        void* p = base ? static_cast<uint8_t*>(base) + off : nullptr;
+        off += pad256(bytes);
+        return p;
+    };
+    BulkBuf b;
+    b.h = static_cast<float*>(take(4 * s.h));
+    b.xq = static_cast<int8_t*>(take(s.xq));
+    b.xd = static_cast<uint32_t*>(take(4 * s.xd));
+    b.qkv = static_cast<float*>(take(4 * s.qkv));
+    const size_t rec = off;
+    b.aq = static_cast<int8_t*>(take(s.aq));
+    b.ad = static_cast<uint32_t*>(take(4 * s.ad));
+    b.dpart = static_cast<float*>(take(4 * s.dpart));
+    b.cand = static_cast<float4*>(take(16 * s.cand));
+    b.rec = reinterpret_cast<float*>(b.aq);
+    b.rec_floats = s.rec;
+    if (base) *B = b;
+    return std::max(off, rec + pad256(4 * s.rec));
+}
+
+int bulk_attn_tokens(size_t room, int NH, int HD, int nsp, int m) {
+    const int fit = std::max<int>(32, (int)std::min<size_t>(kBulkM, room / rec_floats(NH, HD, nsp)) / 32 * 32);
+    if (m <= fit) return m;
+    const int n = (m + fit - 1) / fit;                       // even launches
+    return ((m + n - 1) / n + 31) / 32 * 32;
 }
 
 __device__ __forceinline__ uint16_t f2h_bits(float v) { return __half_as_ushort(__float2half(v)); }
@@ -471,14 +508,14 @@ __global__ __launch_bounds__(kBThreads) void k_bargmax(const float4* cand, int n
 
 // ------------------------------------------------------------------ residual, norm, quant
 // One workgroup per token: h (layer 0: the embedding row) + the down partials in order,
-// written back; RMSNorm and int8 quantisation into the GEMM operand. Thread i holds elements
+// written back; RMSNorm and int8 quantisation into the GEMM operand. prows: rows of one partial. Thread i holds elements
 // 4i .. + 3 (and those 1024 further on); the row meets in LDS, where every wave takes the
 // canonical sum of squares (lane l: elements 256j + 4l + i over j, then i). A wave per token
 // was a chain of its partials' loads on 16 CUs at 64 tokens: 20.4 us with the 10 partials of
 // the 1.5B shape.
 __global__ __launch_bounds__(kBThreads) void k_bnorm(int n, float eps, const float* w, float* h, const float* emb,
-                                                     const int32_t* tok, const float* part, int ks, int8_t* xq,
-                                                     uint32_t* xd) {
+                                                     const int32_t* tok, const float* part, int ks, int prows,
+                                                     int8_t* xq, uint32_t* xd) {
     constexpr int NI = kBMaxE / (4 * kBThreads);
     __shared__ __align__(16) float row[kBMaxE];
     const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
@@ -493,7 +530,7 @@ __global__ __launch_bounds__(kBThreads) void k_bnorm(int n, float eps, const flo
             wv[i] = *reinterpret_cast<const float4*>(w + e);
             if (ks > 0) {
                 const float* pt = part + (size_t)t * n + e;
-                const size_t step = (size_t)kBulkSplitM * n;
+                const size_t step = (size_t)prows * n;
                 float4 s = *reinterpret_cast<const float4*>(pt);
                 auto add = [&](float4 p) {
                     s = make_float4(__fadd_rn(s.x, p.x), __fadd_rn(s.y, p.y), __fadd_rn(s.z, p.z), __fadd_rn(s.w, p.w));
@@ -927,7 +964,7 @@ void launch_bulk(const DModel& M, const DLayer* layers, const BulkBuf& B, int p0
     const int E = M.E, ntt = (m + 63) / 64, nbE = E / 32;
     const int nsp = (p0 + m - 1) / (kAttnChunk * kAttnSplit) + 1;
     auto norm = [&](const float* w, const float* emb, int ks) {
-        LAUNCH(k_bnorm, m, kBThreads, s, E, M.eps, w, B.h, emb, M.tokbuf + p0, B.dpart, ks, B.xq, B.xd);
+        LAUNCH(k_bnorm, m, kBThreads, s, E, M.eps, w, B.h, emb, M.tokbuf + p0, B.dpart, ks, ntt * 64, B.xq, B.xd);
     };
     int ks = 0;                                              // down partials the next norm adds
     for (int l = 0; l < M.NL; l++) {
@@ -940,10 +977,18 @@ void launch_bulk(const DModel& M, const DLayer* layers, const BulkBuf& B, int p0
             const size_t threads = (size_t)m * (M.NH + 2 * M.NKV) * (HD / 2);
             LAUNCH((k_brope<HD>), (unsigned)((threads + kBThreads - 1) / kBThreads), kBThreads, s, B.qkv, L.bqkv, M.rope, M.NH,
                    M.NKV, M.QKV, m, p0, M.maxseq, M.kc + kv, M.vc + kv);
-            LAUNCH((k_battn<HD>), (unsigned)(M.NH * nsp * ((m + kAT - 1) / kAT)), kAThreads, s, B.qkv, M.QKV, M.kc + kv, M.vc + kv,
-                   M.NH, M.G, m, p0, M.maxseq, nsp, M.scale, B.rec, nbE, B.xq, B.xd);
-            if (nsp > 1)
-                LAUNCH((k_bcomb<HD>), (m * M.NH + 3) / 4, kBThreads, s, B.rec, M.NH, m, p0, nsp, nbE, B.xq, B.xd);
+            // all tokens at once, or as many as the split records have room for: q, K/V and the
+            // operand are addressed from the launch's first token
+            const int per = nsp > 1 ? bulk_attn_tokens(B.rec_floats, M.NH, HD, nsp, m) : m;
+            for (int t = 0; t < m; t += per) {
+                const int mt = std::min(per, m - t), ns = (p0 + t + mt - 1) / (kAttnChunk * kAttnSplit) + 1;
+                int8_t* xq = B.xq + bx_at(nbE, t, 0, 0);
+                uint32_t* xd = B.xd + bd_at(nbE, t, 0);
+                LAUNCH((k_battn<HD>), (unsigned)(M.NH * ns * ((mt + kAT - 1) / kAT)), kAThreads, s, B.qkv + (size_t)t * M.QKV,
+                       M.QKV, M.kc + kv, M.vc + kv, M.NH, M.G, mt, p0 + t, M.maxseq, ns, M.scale, B.rec, nbE, xq, xd);
+                if (ns > 1)
+                    LAUNCH((k_bcomb<HD>), (mt * M.NH + 3) / 4, kBThreads, s, B.rec, M.NH, mt, p0 + t, ns, nbE, xq, xd);
+            }
         };
         if (M.HD == 64) attn(std::integral_constant<int, 64>());
         else attn(std::integral_constant<int, 128>());
@@ -955,7 +1000,7 @@ void launch_bulk(const DModel& M, const DLayer* layers, const BulkBuf& B, int p0
         if ((L.gu.rows >> 6) * ntt <= kBulkWgs) gemm<BE_GU>(L.gu, B.xq, B.xd, ntt, 1, nullptr, 0, B.aq, B.ad, s);
         else gemm_w<BE_GU>(L.gu, B.xq, B.xd, ntt, B.aq, B.ad, nullptr, s);
         ks = ntt * 64 <= kBulkSplitM ? L.d.ks : 0;
-        if (ks) gemm<BE_PART>(L.d, B.aq, B.ad, ntt, ks, B.dpart, kBulkSplitM * E, nullptr, nullptr, s);
+        if (ks) gemm<BE_PART>(L.d, B.aq, B.ad, ntt, ks, B.dpart, ntt * 64 * E, nullptr, nullptr, s);
         else gemm<BE_RES>(L.d, B.aq, B.ad, ntt, 1, B.h, 0, nullptr, nullptr, s);
     }
     if (!all && !last) return;

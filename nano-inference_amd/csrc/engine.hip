@@ -48,7 +48,7 @@ struct mi_engine {
     DModel* dM = nullptr;         // device copies the kernels read: [0] M, [1] M_logits, [2] profiling
     DLayer* d_layers = nullptr;
     std::vector<DLayer> layers;   // host copy (the panel launches take the matrices as arguments)
-    BulkBuf bulk{};               // work buffers of the prompt panels
+    BulkBuf bulk{};               // work buffers of the prompt panels (h == nullptr: prompts run in steps)
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int nwg_persistent = 0;       // workgroups of the persistent step kernel (0: per-phase launches)
@@ -325,6 +325,24 @@ static Dims step_dims(int NL, int E, int FF, int NH, int NKV, int V, int maxseq,
     return d;
 }
 
+// the K and V caches: the prompt panels read whole attention chunks, up to a chunk past the last row
+static size_t kv_alloc(const Dims& d) { return lay::kv_size(d) + (size_t)kAttnChunk * d.HD; }
+
+// Work buffers of the prompt panels, for an engine that can run one. The last allocation of a
+// load: where the memory for them is missing, the prompts run in steps.
+static int alloc_bulk(mi_engine* e, const Dims& D) {
+    if (e->opts.tchunk != kMaxT || e->maxseq < kBulkMin) return MI_OK;
+    const BulkSizes s = bulk_sizes(e->E, e->FF, e->NH, e->HD, e->QKV, e->V, e->maxseq, e->ks[3], lay::kv_size(D));
+    void* d = nullptr;
+    const int rc = dev_alloc(e, &d, bulk_bind(s, nullptr, nullptr));
+    if (rc == MI_ERR_OOM) {
+        e->err.clear();
+        return MI_OK;
+    }
+    if (rc == MI_OK) bulk_bind(s, d, &e->bulk);
+    return rc;
+}
+
 static int load_impl(mi_engine* e, const char* path) {
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= e->opts.device)
@@ -495,9 +513,7 @@ static int load_impl(mi_engine* e, const char* path) {
     M.arec = attn_record_floats(e->HD);
     const size_t NL = (size_t)e->NL;
     const Dims D = step_dims(e->NL, e->E, e->FF, e->NH, e->NKV, e->V, e->maxseq, e->cb, e->ks, e->n_cu);
-    // the prompt panels read whole attention chunks: up to a chunk past the last row
-    const size_t kv_pad = (size_t)kAttnChunk * e->HD;
-    if ((rc = alloc_buf(e, &M.kc, lay::kv_size(D) + kv_pad)) || (rc = alloc_buf(e, &M.vc, lay::kv_size(D) + kv_pad)) ||
+    if ((rc = alloc_buf(e, &M.kc, kv_alloc(D))) || (rc = alloc_buf(e, &M.vc, kv_alloc(D))) ||
         (rc = alloc_buf(e, &M.tokbuf, (size_t)e->maxseq + 1)) ||
         (rc = alloc_buf(e, &M.hbuf, lay::hbuf_size(D))) ||
         (rc = alloc_buf(e, &M.qkv_part, lay::qkv_part_size(D))) ||
@@ -521,14 +537,6 @@ static int load_impl(mi_engine* e, const char* path) {
         (rc = alloc_buf(e, &M.dT, lay::dT_size(D))) ||
         (rc = alloc_buf(e, &M.candT, lay::candT_size(D))) || (rc = alloc_buf(e, &M.spec, 1)))
         return rc;
-    // prompt panels (mi_prefill, mi_teacher)
-    const BulkSizes bs = bulk_sizes(e->E, e->FF, e->NH, e->HD, e->QKV, e->V, e->maxseq, e->ks[3]);
-    BulkBuf& B = e->bulk;
-    if ((rc = alloc_buf(e, &B.h, bs.h)) || (rc = alloc_buf(e, &B.xq, bs.xq)) || (rc = alloc_buf(e, &B.xd, bs.xd)) ||
-        (rc = alloc_buf(e, &B.qkv, bs.qkv)) || (rc = alloc_buf(e, &B.aq, bs.aq)) || (rc = alloc_buf(e, &B.ad, bs.ad)) ||
-        (rc = alloc_buf(e, &B.dpart, bs.dpart)) || (rc = alloc_buf(e, &B.rec, bs.rec)) ||
-        (rc = alloc_buf(e, &B.cand, bs.cand)))
-        return rc;
     M.logits = nullptr;
     M.logitsT = nullptr;
     M.prof = nullptr;
@@ -545,6 +553,7 @@ static int load_impl(mi_engine* e, const char* path) {
     if ((rc = alloc_buf(e, &e->M_logits.logits, (size_t)e->V))) return rc;
     if ((rc = alloc_buf(e, &e->M_logits.logitsT, lay::logitsT_size(D)))) return rc;
     if ((rc = alloc_buf(e, &e->dM, 3))) return rc;
+    if ((rc = alloc_bulk(e, D))) return rc;
     HIPCHK(e, hipMemcpy(e->dM, &e->M, sizeof(DModel), hipMemcpyHostToDevice));
     HIPCHK(e, hipMemcpy(e->dM + 1, &e->M_logits, sizeof(DModel), hipMemcpyHostToDevice));
     HIPCHK(e, hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
@@ -696,6 +705,32 @@ int mi_check_layout(const mi_synth_shape* sh, int32_t max_ctx, int32_t n_cu, int
             chk("xT", lay::xT(E, lay::xt_slot(NL, NL, 0)) + (size_t)(t + 1) * lay::xT_tok(E) - 1, lay::xT_size(D));
             chk("logitsT", (size_t)t * V + V - 1, lay::logitsT_size(D));
             for (int w = 0; w < n_cu; w++) chk("candT", lay::candT(w, t) + 3, lay::candT_size(D));
+        }
+    }
+    // a prompt of pos + T tokens in panels (bulk.hip): every buffer's last element
+    if (pos + T >= kBulkMin) {
+        const BulkSizes bs = bulk_sizes(E, FF, NH, HD, QKV, V, D.maxseq, ks[3], lay::kv_size(D));
+        const int n = pos + T, per = bulk_panel_tokens(n);
+        for (int p = 0; p < n; p += per) {
+            const int m = std::min(per, n - p), rows = (m + 63) / 64 * 64;     // the GEMMs' whole tiles
+            chk("panel h", (size_t)rows * E - 1, bs.h);
+            chk("panel xq", bx_at(nbE, rows - 1, nbE - 1, 31), bs.xq);
+            chk("panel xd", bd_at(nbE, rows - 1, nbE - 1), bs.xd);
+            chk("panel qkv", (size_t)rows * QKV - 1, bs.qkv);
+            chk("panel aq", bx_at(nbF, rows - 1, nbF - 1, 31), bs.aq);
+            chk("panel ad", bd_at(nbF, rows - 1, nbF - 1), bs.ad);
+            if (rows <= kBulkSplitM) chk("panel dpart", (size_t)ks[3] * rows * E - 1, bs.dpart);
+            chk("panel cand", (size_t)rows * (V / 64) - 1, bs.cand);
+            const int span = kAttnChunk * kAttnSplit, nsp = (p + m - 1) / span + 1;
+            const int at = nsp > 1 ? bulk_attn_tokens(bs.rec, NH, HD, nsp, m) : m;
+            if (at < m && at % 32) return fail("panel attention of %d tokens: not whole operand tiles", at);
+            for (int t = 0; t < m; t += at) {
+                const int mt = std::min(at, m - t), ns = (p + t + mt - 1) / span + 1;
+                if (ns > 1) chk("panel rec", (size_t)mt * NH * ns * (HD + 4) - 1, bs.rec);
+            }
+            // whole chunks of K and V
+            chk("kc/vc", lay::kv(NKV, D.maxseq, HD, NL - 1, NKV - 1, (p + m + kAttnChunk - 1) / kAttnChunk * kAttnChunk) - 1,
+                kv_alloc(D));
         }
     }
     if (bad) return fail("%s index %zu outside its %zu elements (T=%d pos=%d)", what, at, lim, T, pos);
@@ -936,10 +971,10 @@ static int generate_ring(mi_engine* e, int n_gen, int32_t* out, float* margins, 
 
 // Prompts of kBulkMin tokens and more go through the weights in panels of up to kBulkM
 // tokens (bulk.hip; the same bits). tchunk below its maximum asks for smaller steps and
-// keeps them.
-static bool use_bulk(const mi_engine* e, int n) { return n >= kBulkMin && e->opts.tchunk == kMaxT; }
+// keeps them (no buffers, see alloc_bulk).
+static bool use_bulk(const mi_engine* e, int n) { return n >= kBulkMin && e->bulk.h; }
 static int run_bulk(mi_engine* e, int n, bool all) {
-    const int np = (n + kBulkM - 1) / kBulkM, per = ((n + np - 1) / np + 63) / 64 * 64;   // even panels, whole tiles
+    const int per = bulk_panel_tokens(n);
     for (int p = 0; p < n; p += per) {
         const int m = std::min(per, n - p);
         launch_bulk(e->M, e->layers.data(), e->bulk, p, m, all, p + m == n, e->stream);

@@ -88,3 +88,49 @@ def test_panel_infinite_values_stay_with_their_positions(tmpdir_mi):
     print("[gpu-panel] finite margins", int(fin.sum()), "of", n, flush=True)
     assert 2 <= fin.sum() < n                    # the case has both kinds
     assert np.array_equal(fin, np.isfinite(ma)) and np.array_equal(bits(ma[fin]), bits(mb[fin])) and pa == pb
+
+
+def test_panel_attention_in_several_launches():
+    """contexts whose split records exceed the room kept for them: the attention of a panel goes
+    out in two launches (7 heads of 128 over 9 and 10 splits of 1024 positions)"""
+    path = synth_cached("panel-hd128-cb4", ODD, 31, qk_bias_std=2.0, norm_offset=1.0)
+    n = 9300
+    ids = minfer.prompt_ids(n, n, ODD["n_vocab"])
+    a, b = minfer.Engine(path, max_ctx=9408), minfer.Engine(path, max_ctx=9408, tchunk=7)
+    print("[gpu-panel] long prompt", n, flush=True)
+    pa, ma = a.teacher(ids)
+    pb, mb = b.teacher(ids)
+    assert pa == pb and np.array_equal(bits(ma), bits(mb))
+    fa = a.prefill(ids)
+    assert fa[0] == pb[-1] and bits(fa[1]) == bits(mb[-1])
+    b.prefill(ids)
+    _, _, la = a.step(ids[0], n, want_logits=True)
+    _, _, lb = b.step(ids[0], n, want_logits=True)
+    assert np.array_equal(bits(la), bits(lb))
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("opts,limit", [(dict(max_ctx=8), 12), (dict(max_ctx=64, tchunk=7), 12), (dict(max_ctx=64), 12),
+                                        (dict(max_ctx=131072, tchunk=7), 300), (dict(max_ctx=131072), 400)],
+                         ids=["ctx8", "ctx64-steps", "ctx64", "ctx131072-steps", "ctx131072"])
+def test_panel_buffers_fit_the_engine(opts, limit):
+    """device memory (MB) of a loaded engine: panel buffers only where panels can run and for no
+    more tokens than the context has (2048 tokens' worth of this model's takes 15 MB beside
+    the 6 MB of everything else), and bounded split records in a long context (285 MB for 2048
+    tokens at once, beside 235 MB of K/V and step records)"""
+    import torch
+    path = synth_cached("panel-hd64", TINY, 31, qk_bias_std=2.0, norm_offset=1.0)
+
+    def used(**o):
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        e = minfer.Engine(path, **o)
+        n = free - torch.cuda.mem_get_info()[0]
+        e.close()
+        return n / 1e6
+
+    used(max_ctx=64)                             # what the first load of a process adds
+    mb = used(**opts)
+    print("[gpu-panel] %s: %.1f MB" % (opts, mb), flush=True)
+    assert mb <= limit

@@ -221,3 +221,15 @@ def test_step_indices_stay_inside_their_buffers(name, max_ctx):
     rc, msg = minfer.check_layout(shape, max_ctx, 256, 8, max_ctx - 7)
     assert rc != 0 and "past the context" in msg
 
+
+@pytest.mark.parametrize("name,max_ctx", [("TINY", 9), ("TINY", 64), ("SMALL", 100), ("S05", 777), ("S15", 4352), ("S3", 2049),
+                                          ("S15", 32768), ("S3", 32768), ("TINY", 131072)])
+def test_panel_indices_stay_inside_their_buffers(name, max_ctx):
+    """The prompt panels' part of the same walk (a prompt of pos + T tokens): the last element of
+    every panel buffer, the split records of each attention launch and the whole chunks of K
+    and V past the last row, at the edges of tiles, panels, splits and the context"""
+    shape = LAYOUT_SHAPES[name]
+    for n in sorted({9, 10, 63, 64, 65, 256, 257, 1024, 1025, 2048, 2049, 4095, 9000, max_ctx // 2, max_ctx - 1, max_ctx}):
+        if 9 <= n <= max_ctx:
+            rc, msg = minfer.check_layout(shape, max_ctx, 256, 1, n - 1)
+            assert rc == 0, (name, max_ctx, n, msg)
