@@ -182,8 +182,9 @@ int32_t mi_detok_piece(const char* piece, int32_t len, char* out, int32_t cap);
  * last step `reps` times on the engine stream and returns its mean duration from
  * HIP events. phase: 0 qkv, 1 attention, 2 chunk merge (launched only past 16 chunks),
  * 3 o, 4 gate/up + SiLU + quant, 5 down, 6 lm_head, 7 argmax, 8 the whole persistent
- * step kernel (persistent mode). Needs a completed step; re-running a phase rewrites
- * the same values, so the engine state is unchanged. */
+ * step kernel (persistent mode). Needs a completed step, prefill or teacher run; the
+ * last position's step runs once by phases before (untimed), so that re-running a phase
+ * rewrites the same values and the engine state is unchanged. */
 int mi_time_phase(mi_engine* e, int32_t phase, int32_t layer, int32_t reps, double* avg_ms);
 
 /* In-kernel phase profile of one persistent step (the reference's PROFILE=1,

@@ -1287,6 +1287,9 @@ int mi_time_phase(mi_engine* e, int32_t phase, int32_t layer, int32_t reps, doub
     if (e->cur_len < 1) return set_err(e, MI_ERR_STATE, "mi_time_phase needs a completed step");
     if (phase == 8 && !e->nwg_persistent) return set_err(e, MI_ERR_STATE, "phase 8 is the persistent step kernel");
     const int pos = e->cur_len - 1;
+    // the phase kernels read each other's buffers, which a persistent or multi-token step or a
+    // prompt panel does not leave as they do: one whole step by phases (the same values) first
+    if (phase < 8) launch_step_phases(e->M, e->dM, e->n_cu, pos, 1, e->stream);
     HIPCHK(e, hipEventRecord(e->ev0, e->stream));
     for (int r = 0; r < reps; r++) {
         if (phase == 8) HIPCHK(e, launch_step_persistent(e->M, e->dM, e->nwg_persistent, pos, 1, e->coop, e->stream));

@@ -445,6 +445,26 @@ def test_rewind_and_restep():
     eng.close()
 
 
+@pytest.mark.parametrize("persistent", [2, 0])
+@pytest.mark.parametrize("n", [1, 8, 9, 20])
+def test_time_phase_leaves_the_state(n, persistent):
+    """mi_time_phase re-launches phase kernels of the last position's step and changes nothing,
+    whatever ran it: a single-token step (1), a multi-token step (8) or a panel (9, 20)"""
+    path = synth_cached("eng-256", TINY, 7)
+    ids = minfer.prompt_ids(n, n, TINY["n_vocab"])
+    say("time_phase after a prompt of %d, persistent %d" % (n, persistent))
+    eng = minfer.Engine(path, max_ctx=64, persistent=persistent)
+    eng.prefill(ids)
+    want, wm = eng.generate(12)
+    eng.prefill(ids)
+    for ph in range(8):
+        for layer in range(TINY["n_layer"]):
+            assert eng.time_phase(ph, layer=layer, reps=2) > 0 or ph == 2   # 2: not launched in a short context
+    got, gm = eng.generate(12)
+    assert got == want and np.array_equal(np.float32(gm).view(np.uint32), np.float32(wm).view(np.uint32))
+    eng.close()
+
+
 @pytest.mark.parametrize("mode", ["generate", "generate_cb", "step"])
 def test_barrier_failure_recomputes_cooperatively(mode):
     """The persistent kernel goes out as a plain launch; if a grid barrier gives up
