@@ -60,7 +60,7 @@ typedef struct mi_opts {
                               on); 0: one launch per phase; 2 (default): as 1, and each multi-token
                               step (prompt chunks, verify steps) also one persistent launch, the same
                               bits as its per-phase launches (1), and faster on MI355X: T = 8 verify
-                              2.20 vs 2.25 ms, 512-token prefill 90.2 vs 91.4 ms */
+                              2.20 vs 2.25 ms, 512 prompt tokens in 8-token steps 90.2 vs 91.4 ms */
     int32_t stop_eos;      /* mi_generate stops after tokenizer.ggml.eos_token_id */
     int32_t device;        /* HIP device ordinal */
     int32_t graphs;        /* 1: each multi-token step replays a HIP graph captured once per (T, logits)
@@ -269,24 +269,27 @@ int mi_q4_block_isums(const uint8_t* packed, int32_t rows, int32_t nb, int32_t c
                       const int8_t* xq, int32_t* isum, void* stream);
 
 /* single-query GQA attention over an fp16 cache (cuda_infer.cu:650-702 attn_partial +
- * attn_combine, mega.cu:414-521), two kernel launches on `stream` (chunk records, then
- * their merge), or one up to 512 positions: q[n_head][hd] fp32, kc/vc [n_head_kv][ctx][hd] fp16, positions 0..L-1,
- * out[n_head][hd]; n_head / n_head_kv <= 8, at most 512 splits of 16 64-position chunks
- * (L <= 524288). scratch holds mi_attn_scratch_floats(n_head, hd, L) floats: a record
- * per head and 64-position chunk, written and read within the call (no initial
- * contents needed). Calls that share a scratch buffer must not overlap. */
+ * attn_combine, mega.cu:414-521): q[n_head][hd] fp32, kc/vc [n_head_kv][ctx][hd] fp16,
+ * positions 0..L-1, out[n_head][hd]; n_head / n_head_kv <= 8, at most 512 splits of 16
+ * 64-position chunks (L <= 524288). Two kernel launches on `stream`: a record per head and
+ * 64-position chunk into scratch, then their merge; up to 512 positions (fewer with many
+ * heads) one launch that leaves scratch untouched, with the same bits. scratch holds
+ * mi_attn_scratch_floats(n_head, hd, L) floats, written and read within the call (no
+ * initial contents needed). Calls that share a scratch buffer must not overlap. */
 size_t mi_attn_scratch_floats(int32_t n_head, int32_t hd, int32_t L);
 int mi_attn_decode(const float* q, const uint16_t* kc, const uint16_t* vc, int32_t n_head,
                    int32_t n_head_kv, int32_t hd, int32_t L, int32_t ctx, float scale,
                    float* scratch, float* out, void* stream);
 
-/* The same attention (same arguments, scratch and record layout, same merge) with each
- * chunk's scores and p.v as fp16 matrix-core contractions: q and the probabilities are
- * split into two fp16 parts each (~22 significant bits), K and V are used as stored, the
- * products are exact and accumulate in fp32. Within ~1e-6 relative of mi_attn_decode,
- * not bit-identical to it (the order of the sums inside a matrix instruction is the
- * hardware's). Replaces the same reference kernels (cuda_infer.cu:650-702
- * attn_partial + attn_combine); config-3 tolerance 1e-3 relative. */
+/* The same attention (same arguments, same scratch, record layout and merge where it takes
+ * two launches) with each chunk's scores and p.v as fp16 matrix-core contractions: q and
+ * the probabilities are split into two fp16 parts each (~22 significant bits), K and V are
+ * used as stored, the products are exact and accumulate in fp32. Within ~1e-6 relative of
+ * mi_attn_decode, not bit-identical to it (the order of the sums inside a matrix
+ * instruction is the hardware's). Short contexts (up to 256 positions at hd 128, 512 at
+ * hd 64, fewer with many heads) take mi_attn_decode's one launch, which is faster there:
+ * no matrix cores, its bits, scratch untouched. Replaces the same reference kernels
+ * (cuda_infer.cu:650-702 attn_partial + attn_combine); config-3 tolerance 1e-3 relative. */
 int mi_attn_decode_mfma(const float* q, const uint16_t* kc, const uint16_t* vc, int32_t n_head,
                         int32_t n_head_kv, int32_t hd, int32_t L, int32_t ctx, float scale,
                         float* scratch, float* out, void* stream);

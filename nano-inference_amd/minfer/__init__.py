@@ -396,7 +396,8 @@ def attn_decode(q, kc, vc, n_head, n_head_kv, hd, L, ctx, scale, scratch, out, s
 
 
 def attn_decode_mfma(q, kc, vc, n_head, n_head_kv, hd, L, ctx, scale, scratch, out, stream=None):
-    """attn_decode with MFMA chunk records (mi_attn_decode_mfma): ~1e-6 relative, not bit-identical"""
+    """attn_decode with MFMA chunk records (mi_attn_decode_mfma): ~1e-6 relative, not bit-identical
+    (short contexts run attn_decode's one launch, with its bits)"""
     _check(lib().mi_attn_decode_mfma(_ptr(q), _ptr(kc), _ptr(vc), n_head, n_head_kv, hd, L, ctx, C.c_float(scale),
                                      _ptr(scratch), _ptr(out), _stream(stream)))
 
