@@ -110,11 +110,13 @@ int main(int argc, char** argv) {
         }
         std::printf("\n");
         std::fflush(stdout);
+        // the reference's line; a sequence that ran in panels (minfer.h tchunk) took no such steps, and
+        // the figure is then the time of as many tokens: the last one holds for both
         std::fprintf(stderr,
                      "teacher-forced top-1 agreement: %d/%d | %d positions in %.1f ms (%.2f ms per %d-token step) | "
-                     "logit hash %016llx\n",
+                     "logit hash %016llx | %.3f ms per token\n",
                      agree, total, P, ms, ms * o.tchunk / P, o.tchunk,
-                     (unsigned long long)mi_pred_hash(pred.data(), mg.data(), P));
+                     (unsigned long long)mi_pred_hash(pred.data(), mg.data(), P), ms / P);
         if (env_int("MARGINS", 0))
             for (int i = 0; i < P; i++) std::fprintf(stderr, "%d:%d:%.4f%c", i, pred[i], mg[i], i + 1 < P ? ' ' : '\n');
         mi_free(e);

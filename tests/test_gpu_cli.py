@@ -135,4 +135,7 @@ def test_cli_teacher_mode():
         agree, total, npos, chunk, hsh = int(m.group(1)), int(m.group(2)), int(m.group(3)), int(m.group(4)), m.group(5)
         assert (agree, total, npos, chunk) == (len(seq) - len(prompt), len(seq) - len(prompt), len(seq), tchunk)
         assert int(hsh, 16) == want
+        # 34 tokens at tchunk 8 run as a panel: the time per token holds for panels and steps
+        whole = re.search(r"positions in ([\d.]+) ms .*\| ([\d.]+) ms per token$", err, re.M)
+        assert whole and abs(float(whole.group(2)) - float(whole.group(1)) / npos) <= 0.0011 + 0.05 / npos
         assert out.strip() == b""
