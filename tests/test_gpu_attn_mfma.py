@@ -70,10 +70,14 @@ def check_canon(got, q, k16, v16, nh, nkv, hd, L, scale, f64=False):
 @pytest.mark.parametrize("nh,nkv,hd,L", [(12, 2, 128, 1), (12, 2, 128, 64), (12, 2, 128, 65), (12, 2, 128, 300),
                                          (14, 2, 64, 200), (16, 2, 128, 1024), (4, 2, 64, 130), (2, 2, 128, 77),
                                          (14, 2, 64, 1100), (16, 2, 128, 2049), (8, 1, 128, 5000),
+                                         # matrix-core records with 1 to 5 query heads per kv head
+                                         (2, 2, 128, 257), (3, 3, 64, 513), (4, 2, 64, 640), (4, 2, 128, 600),
+                                         (6, 2, 128, 300), (8, 2, 64, 530), (10, 2, 128, 650), (10, 2, 64, 641),
                                          (32, 4, 64, 32768), (24, 4, 128, 32700), (12, 2, 128, 33000)])
 def test_attention_mfma_vs_canon(torch, nh, nkv, hd, L):
     """every group size G = 1..8, both head sizes, ragged last chunks, one unit per
-    workgroup and several (L = 32768: 1024 units on 512 workgroups)"""
+    workgroup and several (L = 32768: 1024 units on 512 workgroups). Up to 256 positions at
+    head size 128 and 512 at 64 the call runs the canonical one-launch kernel"""
     say("mfma attention nh=%d nkv=%d hd=%d L=%d" % (nh, nkv, hd, L))
     rng = np.random.default_rng(1000 + L + nh)
     ctx = L + 5
@@ -144,7 +148,8 @@ def test_attention_mfma_scratch_reuse(torch):
     canonical entry point: each call writes every record it reads"""
     rng = np.random.default_rng(11)
     scratch = torch.full((minfer.attn_scratch_floats(16, 128, 5000),), float("nan"), device="cuda")
-    for nh, nkv, hd, L in [(12, 2, 128, 3000), (4, 2, 64, 100), (16, 2, 128, 5000), (12, 2, 128, 64)]:
+    for nh, nkv, hd, L in [(12, 2, 128, 3000), (4, 2, 64, 100), (16, 2, 128, 5000), (12, 2, 128, 64), (4, 2, 64, 900),
+                           (12, 2, 128, 600)]:
         say("mfma scratch reuse nh=%d hd=%d L=%d" % (nh, hd, L))
         ctx = L + 3
         q = rng.standard_normal((nh, hd)).astype(np.float32)

@@ -100,7 +100,7 @@ def test_chunked_prefill_equals_single_steps(persistent):
     ids = minfer.prompt_ids(8, 37, TINY["n_vocab"])
     say("chunked prefill, 37-token prompt, persistent=%d" % persistent)
     res = {}
-    for tchunk in (1, 3, 8):
+    for tchunk in (1, 3, 7, 8):      # 8: the prompt runs as a panel
         eng = minfer.Engine(path, max_ctx=128, tchunk=tchunk, persistent=persistent)
         first, mg = eng.prefill(ids)
         a, m, lg = eng.step(first, len(ids), want_logits=True)
@@ -109,7 +109,7 @@ def test_chunked_prefill_equals_single_steps(persistent):
         eng.close()
         res[tchunk] = (first, int(bits(mg)), a, int(bits(m)), bits(lg).tobytes(), toks, bits(mgs).tobytes())
         say("tchunk %d: prefill %.2f ms" % (tchunk, st["prefill_ms"]))
-    assert res[3] == res[1] and res[8] == res[1]
+    assert res[3] == res[1] and res[7] == res[1] and res[8] == res[1]
 
 
 def test_cli_teacher_mode():

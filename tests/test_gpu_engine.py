@@ -299,7 +299,7 @@ def test_nan_logits_give_token_zero(tmp_path, mode):
 def test_teacher_forcing_exact(shape, seed):
     """Teacher forcing (mega.cu:857-862, 1192-1205): every position's prediction and
     margin bit-identical to the q8act oracle fed the same ids; the exactness hash the same
-    for prompt chunks of 1, 3 and 8 tokens in both step modes; fed the engine's own
+    for prompt chunks of 1, 3 and 7 tokens and a panel (8) in both step modes; fed the engine's own
     greedy continuation, the top-1 agreement past the prompt is total."""
     path = synth_cached("eng-%d" % shape["n_embd"], shape, seed)
     V = shape["n_vocab"]
@@ -308,7 +308,7 @@ def test_teacher_forcing_exact(shape, seed):
     runs = {}
     plan = None
     for persistent in (1, 0):
-        for tchunk in (1, 3, 8):
+        for tchunk in (1, 3, 7, 8):
             eng = minfer.Engine(path, max_ctx=128, persistent=persistent, tchunk=tchunk)
             plan = plan_of(eng)
             runs[(persistent, tchunk)] = eng.teacher(seq)
@@ -502,20 +502,22 @@ def test_barrier_failure_recomputes_cooperatively(mode):
 
 
 @pytest.mark.parametrize("graphs", [0, 1], ids=["direct", "graphs"])
-@pytest.mark.parametrize("mode", ["multi_step", "prefill", "spec_device"])
+@pytest.mark.parametrize("mode", ["multi_step", "prefill", "prefill_panel", "spec_device"])
 def test_barrier_failure_multi_token_persistent(mode, graphs):
     """The same fallback for the persistent multi-token kernel (persistent=2), with its
     launches direct or replayed from captured graphs: after the host raises the barrier
     flag the engine switches to cooperative launches (graphs captured with plain
     launches are dropped, cooperative launches are never captured) and recomputes, so
-    a multi-token step, a chunked prefill and a speculative generation driven on the
+    a multi-token step, a chunked prefill (tchunk 7: at 8 it would be a panel, which has no
+    grid barrier and only finds the flag raised) and a speculative generation driven on the
     device all equal an undisturbed run's."""
     path = synth_cached("eng-512", SMALL, 21)
     V = SMALL["n_vocab"]
     ids = minfer.prompt_ids(17, 20, V)
     pat = minfer.prompt_ids(5, 6, V)
     rep = (pat * 5)[:28]
-    opts = dict(max_ctx=128, persistent=2, graphs=graphs, spec=2 if mode == "spec_device" else 0)
+    opts = dict(max_ctx=128, persistent=2, graphs=graphs, spec=2 if mode == "spec_device" else 0,
+                tchunk=7 if mode == "prefill" else 8)
 
     def run(eng, flag):
         if mode == "multi_step":
@@ -526,9 +528,9 @@ def test_barrier_failure_multi_token_persistent(mode, graphs):
                 eng.debug_flag_barrier()
             a, m = eng.step(toks[8:], len(ids) + 8)  # ... and replayed here
             return a, m
-        if mode == "prefill":
+        if mode.startswith("prefill"):
             if flag:
-                eng.prefill(ids[:9])                 # 8 + 1 tokens: captures the T = 8 launch
+                eng.prefill(ids[:9])                 # prefill: 7 + 2 tokens, captures both launches
                 eng.debug_flag_barrier()
             f, m = eng.prefill(ids)
             return [f], [m]

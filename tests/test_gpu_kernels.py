@@ -120,6 +120,9 @@ def test_gemv_bit_exact(torch, rows, n_in, cb, ks):
                                          (12, 2, 128, 128), (12, 2, 128, 129), (16, 2, 128, 257), (8, 1, 128, 512),
                                          (12, 2, 128, 513), (14, 2, 64, 1), (14, 2, 64, 63), (3, 3, 64, 512),
                                          (14, 2, 64, 513),
+                                         # record kernels with 1 to 5 query heads per kv head
+                                         (2, 2, 128, 577), (3, 3, 64, 513), (4, 2, 64, 640), (4, 2, 128, 600),
+                                         (6, 2, 128, 700), (8, 2, 64, 530), (10, 2, 128, 650), (10, 2, 64, 641),
                                          (32, 4, 64, 32768), (24, 4, 128, 32700), (12, 2, 128, 33000)])
 def test_attention_bit_exact(torch, nh, nkv, hd, L):
     """chunked attention vs the oracle's canonical order; the last three cases give
@@ -213,11 +216,11 @@ def attention_case(torch, nh, nkv, hd, L, scratch, rng):
 def test_attention_scratch_reuse(torch):
     """one scratch buffer, NaN-filled once, through calls of different shapes: every
     record a call reads it wrote itself, so neither the initial contents nor an earlier
-    call's records change the result"""
+    call's records change the result (up to 512 positions a call leaves the scratch alone)"""
     rng = np.random.default_rng(5)
     scratch = torch.full((minfer.attn_scratch_floats(16, 128, 5000),), float("nan"), device="cuda")
     for nh, nkv, hd, L in [(12, 2, 128, 3000), (4, 2, 64, 100), (12, 2, 128, 3000), (16, 2, 128, 5000),
-                           (14, 2, 64, 1100), (12, 2, 128, 64)]:
+                           (14, 2, 64, 1100), (12, 2, 128, 64), (4, 2, 64, 900), (12, 2, 128, 600)]:
         say("scratch reuse nh=%d hd=%d L=%d" % (nh, hd, L))
         attention_case(torch, nh, nkv, hd, L, scratch, rng)
 

@@ -198,10 +198,10 @@ def test_graph_replays_equal_direct_launches(persistent):
     path = synth_cached("eng-512", SMALL, 21)
     V = SMALL["n_vocab"]
     prompt = minfer.prompt_ids(5, 100, V)
-    g = minfer.Engine(path, max_ctx=256, graphs=1, persistent=persistent)
+    g = minfer.Engine(path, max_ctx=256, graphs=1, persistent=persistent, tchunk=7)
     d = minfer.Engine(path, max_ctx=256, graphs=0, persistent=1)
     for e in (g, d):
-        e.prefill(prompt)            # 12 replays of the T=8 graph and one of T=4 in g
+        e.prefill(prompt)            # 14 replays of the T=7 graph and one of T=2 in g, a panel in d
     cases = [(100, 8, True), (100, 8, False), (64, 5, True), (69, 8, True), (60, 8, False), (68, 2, True),
              (70, 8, True), (70, 8, True)]
     for i, (pos, T, want) in enumerate(cases):

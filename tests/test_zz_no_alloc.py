@@ -3,7 +3,8 @@ mi_attn_decode with a caller-allocated workspace, through the C ABI.
 
 Bar: bit-identical outputs (both run the same kernel over the same records), on
 two calls in a row, the second with a smaller input, so the shared library-held
-scratch is reused with the previous call's contents in it; a shape whose scratch
+scratch is reused with the previous call's contents in it (past 512 positions: shorter
+calls do not touch it); a shape whose scratch
 would exceed the library's fixed size is rejected with a clear error.
 """
 import math
@@ -46,7 +47,8 @@ def run_both(torch, rng, nh, nkv, hd, L):
 
 
 @pytest.mark.parametrize("first,second", [((12, 2, 128, 32768), (12, 2, 128, 4000)),
-                                          ((14, 2, 64, 20000), (4, 2, 64, 130))])
+                                          ((14, 2, 64, 20000), (4, 2, 64, 130)),
+                                          ((14, 2, 64, 20000), (4, 2, 64, 1300))])
 def test_noalloc_matches_workspace_entry(torch, first, second):
     rng = np.random.default_rng(first[3])
     for shape in (first, second):
@@ -99,5 +101,5 @@ def test_noalloc_graph_capture(torch):
         got = out.cpu().numpy()
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), rep
         # eager work on the same scratch between replays (a smaller shape)
-        minfer.attn_decode_noalloc(q[:4].contiguous(), kc, vc, 4, nkv, hd, 500, ctx, scale, other[:4 * hd])
+        minfer.attn_decode_noalloc(q[:4].contiguous(), kc, vc, 4, nkv, hd, 700, ctx, scale, other[:4 * hd])
         torch.cuda.synchronize()
