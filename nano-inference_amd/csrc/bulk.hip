@@ -4,7 +4,7 @@
 //
 // A prompt in 8-token steps reads the weights once per 8 tokens and pays ~291 grid barriers
 // per step: 1.4 ms a step on the 1.5B shape, 84.1 ms for 512 tokens, 530 ms for 3001. Panels
-// read them once: 4.5 and 29.9 ms.
+// read them once per 2048 tokens: 4.5 and 29.9 ms.
 //
 // Every value equals the single-token step's bit for bit (the reduction plan at the top of
 // kernels.hip):
@@ -996,7 +996,7 @@ void launch_bulk(const DModel& M, const DLayer* layers, const BulkBuf& B, int p0
         norm(L.fn, nullptr, 0);
         // K split while the 64 x 64 tiles are about one per CU (us, split / whole K, at 152 and 280
         // row groups: 64 tokens 7.4 / 12.0 and 18.1 / 21.1; 128 tokens 13.9 / 13.0 and 28.6 / 24.3;
-        // 512 tokens 32.5 / 26.9 and 73.5 / 56.5)
+        // 512 tokens 32.5 / 26.9 and 73.5 / 56.5); not measured at the 344 of the 3B shape
         if ((L.gu.rows >> 6) * ntt <= kBulkWgs) gemm<BE_GU>(L.gu, B.xq, B.xd, ntt, 1, nullptr, 0, B.aq, B.ad, s);
         else gemm_w<BE_GU>(L.gu, B.xq, B.xd, ntt, B.aq, B.ad, nullptr, s);
         ks = ntt * 64 <= kBulkSplitM ? L.d.ks : 0;
