@@ -2755,7 +2755,8 @@ __global__ __launch_bounds__(64) void k_isums(PMat W, const int8_t* xq, int32_t*
 // q[nh][hd] fp32 and an fp16 cache [nkv][ctx][hd]; two launches do the whole
 // attention: k_attn_rec writes a record (o[hd], m, l) per head and 64-position chunk,
 // k_attn_merge merges them in the canonical order. scratch: chunk records o
-// [nh][nch][hd], m [nh][nch], l [nh][nch].
+// [nh][nch][hd], m [nh][nch], l [nh][nch]. Short contexts take one launch and no scratch
+// (k_attn_one, attn_one_takes).
 constexpr int kAttnMaxG = 8;        // query heads per kv head
 
 // Standalone attention, part 1: the chunk records. A unit is (kv head, 64-position
@@ -2840,9 +2841,9 @@ __global__ __launch_bounds__(64 * (S * ((kAttnMaxG + H - 1) / H) + 1)) void k_at
 }
 
 // Standalone attention of a short context in one launch: one workgroup per query head, wave c
-// on chunk c (up to kOneChunks). K comes by DMA into the wave's swizzled tile; V is not shared between waves, so a lane loads its dims of all 64 rows
-// straight into registers, everything in flight at once. The chunk arithmetic is
-// attn_core_h's, the merge the canonical one of up to kOneChunks chunks. The query heads of a kv
+// on chunk c (up to kOneChunks). K comes by DMA into the wave's swizzled tile; V is not shared
+// between waves, so a lane loads its dims of all 64 rows straight into registers, everything
+// in flight at once. The chunk arithmetic is attn_core_h's, the merge the canonical one of up to kOneChunks chunks. The query heads of a kv
 // head read its rows from the L2 (which calls take it, and the times: attn_one_takes).
 constexpr int kOneChunks = 8, kOneChunksMx128 = 4;            // (against k_attn_mx at hd 128)
 constexpr int kOneHeadDims = 131072;
